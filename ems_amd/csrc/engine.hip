@@ -136,16 +136,6 @@ __device__ __forceinline__ float coefg(const Lane &L, size_t r, int k, int nz, s
   return rows[(size_t)((const GAS uint32_t *)L.index)[r] * nz + k];
 }
 
-// The block of a one-dimensional launch of gx * nch blocks that takes
-// block b's place, so that each XCD runs a contiguous share of the
-// (row block, x chunk) pairs: a launch hands its blocks to the 8 XCDs in
-// turn (block b to XCD b % 8), so block b + 1, whose rows neighbour block
-// b's, would otherwise run beside another L2. A bijection of [0, nb).
-__device__ __forceinline__ int xcd_contiguous(int b, int nb) {
-  const int per = nb / 8, rem = nb % 8, x = b % 8, q = b / 8;
-  return (x < rem ? x * (per + 1) : rem * (per + 1) + (x - rem) * per) + q;
-}
-
 // Faraday update (kernel.rs:443-511, 566-618): plane-wise in x, all three
 // components at node (i, j, k); padding entries are never written.
 template <bool OE>
@@ -502,10 +492,7 @@ __device__ __forceinline__ size_t cpml_index(const FSlab &s, int i, int j, int k
 // instead of seven for the whole tiled kernel, and measured slower on the
 // 512^3 CPML box (2.976 against 2.849 ms per launch; with 2 slots 2.949).
 //
-// INPLACE (the unfused kernels, which compute each node once): the psi of
-// parity `par` is read and written (the fused kernel's halo recompute reads
-// one buffer and writes the other).
-template <bool ESIDE, bool INPLACE = false>
+template <bool ESIDE>
 __device__ __forceinline__ void cpml_node(const FSlab *__restrict__ slabs, uint32_t mask, int par,
                                           bool write_psi, int i, int j, int k, float d01,
                                           float d02, float d10, float d12, float d20, float d21,
@@ -520,7 +507,7 @@ __device__ __forceinline__ void cpml_node(const FSlab *__restrict__ slabs, uint3
     const int z = cpml_depth(s, i, j, k);
     const size_t qq = cpml_index(s, i, j, k);
     const GAS float *pin = (const GAS float *)((ESIDE || par == 0) ? s.psi0 : s.psi1);
-    GAS float *pout = (GAS float *)((ESIDE || par == (INPLACE ? 0 : 1)) ? s.psi0 : s.psi1);
+    GAS float *pout = (GAS float *)((ESIDE || par == 1) ? s.psi0 : s.psi1);
     float ps;
     cpml_apply<ESIDE>(s, pin[qq], ((const GAS float *)s.b)[z], ((const GAS float *)s.a)[z],
                       ((const GAS float *)s.k)[z], d01, d02, d10, d12, d20, d21, cf0, cf1, cf2, t0,
@@ -529,185 +516,381 @@ __device__ __forceinline__ void cpml_node(const FSlab *__restrict__ slabs, uint3
   }
 }
 
-// ---- unfused H and E updates, software pipelined along x ----
+// ---- unfused H and E updates, four nodes of a z row per thread ----
 //
-// The same updates (same expressions, same values written) with a thread
-// marching a chunk of x-planes and the next plane's inputs loaded before
-// the present plane is computed, so the loads of one plane overlap the
-// arithmetic and stores of the one before. Every load address is valid
-// (neighbours past the grid's end fall back to the node itself; those
-// values are not used).
+// A thread owns a quad of four consecutive nodes of one z row (rows of nz
+// nodes are cut into ceil(nz / 4) quads, the last one short). Every field,
+// coefficient and psi access is one 16-byte load or store per thread (rows
+// start at any 4-byte boundary; global accesses take that), so a wave moves
+// 1 KiB per instruction, and the index arithmetic, coefficient row lookups
+// and CPML slab tests are paid once per four nodes. Loads may run up to
+// three floats past a row (into the next row or the allocations' padding):
+// those values are not used.
 //
-// CP: the side's CPML slabs (the fused kernel's slab table, every slab of
-// the side in it) corrected here, after the update, in registration order
-// with the very expressions of cpml_slab, instead of in launches of their
-// own; a plane that a slab's x range holds stores all three components.
+// Bound by memory: 36 bytes per node and half-step plus 4 per dense lane
+// (513^3 nodes with CPML: H 1.29 ms, E 1.31 ms, 5.0 TB/s of algorithmic
+// bytes; the kernels before, a node per thread marching 8 x-planes with the
+// next plane loaded ahead, 2.7 TB/s and the H slabs in 12 launches). A
+// thread takes one plane: marching 2 to 64 planes with the shared plane
+// kept in registers measured slower at every size (2.91 to 3.86 ms against
+// 2.61; 72 VGPRs without the march, 120 with it).
+//
+// CP: the side's CPML slabs corrected here, after the update, in
+// registration order with the very expressions of cpml_slab, instead of in
+// launches of their own (513^3 nodes: 0.1 ms per half-step for 9 % of the
+// nodes; the psi loads are issued with the fields').
+constexpr int QW = 5;  // waves per SIMD the quad kernels are held to (90 VGPRs with CPML)
+constexpr size_t QUAD_PAD = 4;  // floats of padding behind (psi: around) quad-read arrays
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 
-// The slabs (bits of the first `nslab` table entries) whose (j, k) box
-// meets the block's nodes p0..p1 of a plane: rows p0/nz..p1/nz and, over
-// one row, its columns (else every column).
-__device__ __forceinline__ uint32_t block_slabs(const FSlab *__restrict__ slabs, int nslab,
-                                                int p0, int p1, int nz) {
-  const int j0 = p0 / nz, j1 = p1 / nz;
-  const int k0 = j0 == j1 ? p0 - j0 * nz : 0, k1 = j0 == j1 ? p1 - j1 * nz : nz - 1;
-  uint32_t m = 0;
-  for (int q = 0; q < nslab; q++) {
-    const FSlab s = cload(slabs, q);
-    if (s.lo1 <= j1 && j0 < s.hi1 && s.lo2 <= k1 && k0 < s.hi2) m |= 1u << q;
+__device__ __forceinline__ f4 ld4(const float *base, unsigned boff) {
+  return *(const GAS f4u *)((const GAS char *)base + boff);
+}
+__device__ __forceinline__ float ld1(const float *base, unsigned boff) {
+  return *(const GAS float *)((const GAS char *)base + boff);
+}
+__device__ __forceinline__ void st4(float *base, unsigned boff, f4 v) {
+  *(GAS f4u *)((GAS char *)base + boff) = v;
+}
+// The first ne elements of a quad.
+__device__ __forceinline__ void st_quad(float *base, unsigned boff, f4 v, int ne) {
+  if (ne >= 4) {
+    st4(base, boff, v);
+  } else {
+    GAS float *p = (GAS float *)((GAS char *)base + boff);
+    p[0] = v[0];
+    if (ne > 1) p[1] = v[1];
+    if (ne > 2) p[2] = v[2];
   }
-  return m;
 }
 
-// The fold's tables: the slab table, per x-plane the slabs (H, E) whose x
-// range holds it, the table's length and the H psi parity.
-struct CpmlIn {
-  const FSlab *slabs;
-  const uint32_t *pmask;
-  int nslab, par;
+// The coefficients of a quad: lane L at plane i (node offset ip), row j,
+// byte offset vo within the plane and node k0 within the row.
+__device__ __forceinline__ f4 coef4(const Lane &L, size_t ip, size_t r, unsigned vo, int k0,
+                                    int nz) {
+  if (L.rows == nullptr) return f4{0.0f, 0.0f, 0.0f, 0.0f};
+  if (L.index == nullptr) return ld4(L.rows + ip, vo);
+  const size_t row = ((const GAS uint32_t *)L.index)[r];
+  return *(const GAS f4u *)((const GAS float *)L.rows + row * nz + k0);
+}
+
+// The quads of a plane in thread order. The nm = nq - ql - qh middle quads
+// of every row come first, row by row, then (from the next block on) the ql
+// first and qh last quads, those that z-normal CPML slabs reach: so the
+// slabs' code runs in waves that hold nothing else instead of in a few
+// lanes of most waves.
+struct QuadGeom {
+  int nx, ny, nz, ql, qh, nm;
+  int gm;     // blocks of 256 threads over the middle quads
+  int gx;     // all blocks of a plane
+  int run;    // consecutive blocks an XCD takes at a time
 };
 
-// What the H update of one node reads (kernel.rs:443-511).
-struct HNode {
-  float uxc, uyn, uzn, ix, iy, iz, uz_j1, uy_k1, ux_k1, ux_j1;
-  float da[3], db[3];
-};
+// Plane and in-plane block of this block. Blocks go round-robin to the 8
+// XCDs; each XCD takes `run` consecutive blocks of the grid at a time.
+__device__ __forceinline__ bool quad_block(const QuadGeom &g, int &i, int &bx) {
+  unsigned b = blockIdx.x;
+  const unsigned w = 8u * (unsigned)g.run, q = b % w;
+  b = b - q + (q % 8u) * (unsigned)g.run + q / 8u;
+  i = (int)(b / (unsigned)g.gx);
+  bx = (int)(b - (unsigned)i * (unsigned)g.gx);
+  return i < g.nx;
+}
 
-__device__ __forceinline__ void h_node_load(HNode &q, const Fields &f, const Lanes &L, size_t o,
-                                            size_t r, int k, int nz, size_t plane, bool iv,
-                                            bool jv, bool kv) {
-  const GAS float *ux = (const GAS float *)f.u[0], *uy = (const GAS float *)f.u[1];
-  const GAS float *uz = (const GAS float *)f.u[2];
-  const size_t oi = iv ? o + plane : o, oj = jv ? o + nz : o, ok = kv ? o + 1 : o;
-  q.uxc = ux[o], q.uyn = uy[oi], q.uzn = uz[oi];
-  q.ix = ((const GAS float *)f.i[0])[o], q.iy = ((const GAS float *)f.i[1])[o];
-  q.iz = ((const GAS float *)f.i[2])[o];
-  q.uz_j1 = uz[oj], q.ux_j1 = ux[oj], q.uy_k1 = uy[ok], q.ux_k1 = ux[ok];
+// Row and first node of block bx's thread; false past the end.
+__device__ __forceinline__ bool quad_at(const QuadGeom &g, int bx, int &j, int &k0) {
+  const bool mid = bx < g.gm;
+  const int w = mid ? g.nm : g.ql + g.qh;  // quads per row of this part (>= 1)
+  const int t = (mid ? bx : bx - g.gm) * 256 + (int)threadIdx.x;
+  j = t / w;
+  int q = t - j * w;
+  if (mid) q += g.ql;
+  else if (q >= g.ql) q += g.nm;
+  k0 = 4 * q;
+  return j < g.ny;
+}
+
+// The CPML slabs of one side as the quad kernels take them, by value: for
+// each component its two normals (ascending), each with at most one slab at
+// the low and one at the high end. Such slabs span the component's whole
+// extent in the other two directions (quad_cpml checks this, and that the
+// corrections of a component come in the order of its normals; other slabs
+// are corrected by launches of their own). An absent end has hi <= lo.
+struct CpmlEnd {
+  float *psi;        // box (i, j, k) order
+  const float *bak;  // b, a, k by depth, each (hi - lo) + 2 QUAD_PAD apart
+  int lo, hi;        // along the normal
+};
+struct QuadCpml {
+  CpmlEnd e[3][2][2];  // component, which of its normals, low / high end
+};
+constexpr int pair_of(int c, int n) { return c == 0 ? n - 1 : (c == 1 ? n / 2 : n); }
+
+// One (component, normal) pair at a quad: whether it is inside an end's
+// slab, and that end's psi quad and coefficient table.
+struct QuadPair {
+  bool in;
+  int lo, hi;
+  GAS float *psi;
+  const float *bak;
+};
+template <bool ESIDE, int C, int N>
+__device__ __forceinline__ QuadPair quad_pair(const QuadCpml &cp, const QuadGeom &g, int i, int j,
+                                              int k0) {
+  const CpmlEnd &A = cp.e[C][pair_of(C, N)][0], &B = cp.e[C][pair_of(C, N)][1];
+  const int ex = g.nx - ((ESIDE == (C == 0)) ? 1 : 0);
+  const int ey = g.ny - ((ESIDE == (C == 1)) ? 1 : 0), ez = g.nz - ((ESIDE == (C == 2)) ? 1 : 0);
+  QuadPair q;
+  const int pos = N == 0 ? i : (N == 1 ? j : k0);
+  const bool hi = N == 2 ? pos + 4 > B.lo : pos >= B.lo;
+  q.lo = hi ? B.lo : A.lo, q.hi = hi ? B.hi : A.hi;
+  q.in = N == 2 ? (pos + 4 > q.lo && pos < q.hi) : (pos >= q.lo && pos < q.hi);
+  q.in = q.in && (N == 0 || i < ex) && (N == 1 || j < ey) && (N == 2 || k0 < ez);
+  q.bak = hi ? B.bak : A.bak;
+  GAS float *psi = (GAS float *)(hi ? B.psi : A.psi);
+  if (N == 0) psi += (ptrdiff_t)((size_t)(i - q.lo) * ey) * ez + (j * ez + k0);
+  if (N == 1) psi += (ptrdiff_t)((size_t)i * (q.hi - q.lo) + (j - q.lo)) * ez + k0;
+  if (N == 2) psi += (ptrdiff_t)((size_t)i * ey + j) * (q.hi - q.lo) + (k0 - q.lo);
+  q.psi = psi;
+  return q;
+}
+
+template <bool ESIDE, int C, int N>
+__device__ __forceinline__ f4 quad_psi(const QuadCpml &cp, const QuadGeom &g, int i, int j,
+                                       int k0) {
+  const QuadPair q = quad_pair<ESIDE, C, N>(cp, g, i, j, k0);
+  f4 p = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (q.in) p = *(const GAS f4u *)q.psi;
+  return p;
+}
+
+// The pair's correction of a quad (cpml.rs:495-543): component t with
+// coefficient cf, d the derivative's difference h - l, pin its psi.
+// Elements outside the slab keep their value and psi.
+template <bool ESIDE, int C, int N>
+__device__ __forceinline__ void quad_cpml_apply(const QuadCpml &cp, const QuadGeom &g, int i,
+                                                int j, int k0, f4 pin, f4 d, f4 cf, f4 &t) {
+  const QuadPair q = quad_pair<ESIDE, C, N>(cp, g, i, j, k0);
+  if (!q.in) return;
+  const int D = q.hi - q.lo + 2 * (int)QUAD_PAD;
+  f4 bz, az, kz;
+  if (N == 2) {
+    const GAS float *b = (const GAS float *)q.bak + (k0 - q.lo);
+    bz = *(const GAS f4u *)b, az = *(const GAS f4u *)(b + D), kz = *(const GAS f4u *)(b + 2 * D);
+  } else {
+    float b1, a1, k1;
+    if (N == 0) {
+      const float *b = q.bak + (i - q.lo);
+      b1 = cload(b), a1 = cload(b, D), k1 = cload(b, 2 * D);
+    } else {
+      const GAS float *b = (const GAS float *)q.bak + (j - q.lo);
+      b1 = b[0], a1 = b[D], k1 = b[2 * D];
+    }
+    bz = f4{b1, b1, b1, b1}, az = f4{a1, a1, a1, a1}, kz = f4{k1, k1, k1, k1};
+  }
+  const float sign = N == (C + 1) % 3 ? 1.0f : -1.0f, scale = ESIDE ? 1.0f : -1.0f;
+  const int ez = g.nz - ((ESIDE == (C == 2)) ? 1 : 0);
+  const int k_lo = N == 2 ? q.lo : 0, k_hi = N == 2 ? q.hi : ez;
+  f4 ps;
 #pragma unroll
-  for (int a = 0; a < 3; a++) {
-    q.da[a] = coefg(L.l[6 + a], r, k, nz, o);
-    q.db[a] = coefg(L.l[9 + a], r, k, nz, o);
+  for (int e = 0; e < 4; e++) {
+    const float sv = sign * d[e];
+    ps[e] = flush(bz[e] * pin[e] + az[e] * sv);
+    const float tn = flush(t[e] + scale * cf[e] * (kz[e] * sv + ps[e]));
+    t[e] = (k0 + e >= k_lo && k0 + e < k_hi) ? tn : t[e];
+  }
+  if (k0 >= k_lo && k0 + 4 <= k_hi) {
+    *(GAS f4u *)q.psi = ps;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      if (k0 + e >= k_lo && k0 + e < k_hi) q.psi[e] = ps[e];
+  }
+}
+
+// Which normals' slabs a wave meets: x by plane, y and z by its quads
+// (every lane of the wave calls it, lanes past the end with in = false).
+template <bool ESIDE>
+__device__ __forceinline__ void quad_normals(const QuadCpml &cp, const QuadGeom &g, bool in, int i,
+                                             int j, int k0, bool &fy, bool &fz) {
+  fy = __any(in && (quad_pair<ESIDE, 0, 1>(cp, g, i, j, k0).in ||
+                    quad_pair<ESIDE, 2, 1>(cp, g, i, j, k0).in));
+  fz = __any(in && (quad_pair<ESIDE, 0, 2>(cp, g, i, j, k0).in ||
+                    quad_pair<ESIDE, 1, 2>(cp, g, i, j, k0).in));
+}
+__device__ __forceinline__ bool quad_x_slab(const QuadCpml &cp, int i) {
+  bool in = false;
+#pragma unroll
+  for (int c = 1; c < 3; c++)
+#pragma unroll
+    for (int e = 0; e < 2; e++) in = in || (i >= cp.e[c][0][e].lo && i < cp.e[c][0][e].hi);
+  return in;
+}
+
+// The psi of the first normal whose slabs the wave meets (two components),
+// loaded with the plane's fields so that the latencies overlap; the other
+// normals' (at the grid's edges and corners) are loaded when their turn
+// comes.
+template <bool ESIDE>
+__device__ __forceinline__ void quad_psi_first(const QuadCpml &cp, const QuadGeom &g, bool fx,
+                                               bool fy, int i, int j, int k0, f4 P[2]) {
+  if (fx) {
+    P[0] = quad_psi<ESIDE, 1, 0>(cp, g, i, j, k0);
+    P[1] = quad_psi<ESIDE, 2, 0>(cp, g, i, j, k0);
+  } else if (fy) {
+    P[0] = quad_psi<ESIDE, 0, 1>(cp, g, i, j, k0);
+    P[1] = quad_psi<ESIDE, 2, 1>(cp, g, i, j, k0);
+  } else {
+    P[0] = quad_psi<ESIDE, 0, 2>(cp, g, i, j, k0);
+    P[1] = quad_psi<ESIDE, 1, 2>(cp, g, i, j, k0);
+  }
+}
+
+// Every correction of a quad; d<c><n> the difference along normal n that
+// component c uses.
+template <bool ESIDE>
+__device__ __forceinline__ void quad_cpml(const QuadCpml &cp, const QuadGeom &g, bool fx, bool fy,
+                                          bool fz, int i, int j, int k0, const f4 P[2],
+                                          const f4 &d01, const f4 &d02, const f4 &d10,
+                                          const f4 &d12, const f4 &d20, const f4 &d21,
+                                          const f4 cf[3], f4 t[3]) {
+  if (fx) {
+    quad_cpml_apply<ESIDE, 1, 0>(cp, g, i, j, k0, P[0], d10, cf[1], t[1]);
+    quad_cpml_apply<ESIDE, 2, 0>(cp, g, i, j, k0, P[1], d20, cf[2], t[2]);
+  }
+  if (fy) {
+    f4 p0 = P[0], p1 = P[1];
+    if (fx) {
+      p0 = quad_psi<ESIDE, 0, 1>(cp, g, i, j, k0);
+      p1 = quad_psi<ESIDE, 2, 1>(cp, g, i, j, k0);
+    }
+    quad_cpml_apply<ESIDE, 0, 1>(cp, g, i, j, k0, p0, d01, cf[0], t[0]);
+    quad_cpml_apply<ESIDE, 2, 1>(cp, g, i, j, k0, p1, d21, cf[2], t[2]);
+  }
+  if (fz) {
+    f4 p0 = P[0], p1 = P[1];
+    if (fx || fy) {
+      p0 = quad_psi<ESIDE, 0, 2>(cp, g, i, j, k0);
+      p1 = quad_psi<ESIDE, 1, 2>(cp, g, i, j, k0);
+    }
+    quad_cpml_apply<ESIDE, 0, 2>(cp, g, i, j, k0, p0, d02, cf[0], t[0]);
+    quad_cpml_apply<ESIDE, 1, 2>(cp, g, i, j, k0, p1, d12, cf[1], t[1]);
   }
 }
 
 template <bool OE, bool CP>
-__global__ void __launch_bounds__(256) h_update_pf(Fields f, Lanes L, int nx, int ny, int nz,
-                                                   int chunk, CpmlIn cp) {
-  const int plane = ny * nz, gx = (plane + 255) / 256;
-  const int b = xcd_contiguous(blockIdx.x, gridDim.x);
-  const int p = (b % gx) * blockDim.x + threadIdx.x;
-  const uint32_t mblk =
-      CP ? block_slabs(cp.slabs, cp.nslab, (b % gx) * 256, min((b % gx) * 256 + 255, plane - 1), nz)
-         : 0u;
-  if (p >= plane) return;
-  const int j = p / nz, k = p - j * nz;
-  const int i0 = (b / gx) * chunk;
-  const int i1 = min(nx, i0 + chunk);
-  const bool jv = j < ny - 1, kv = k < nz - 1;
-  GAS float *ix = (GAS float *)f.i[0], *iy = (GAS float *)f.i[1], *iz = (GAS float *)f.i[2];
-  size_t o = (size_t)i0 * plane + p;
-  float uyc = ((const GAS float *)f.u[1])[o], uzc = ((const GAS float *)f.u[2])[o];
-  HNode cur, nxt;
-  h_node_load(cur, f, L, o, (size_t)i0 * ny + j, k, nz, plane, i0 + 1 < nx, jv, kv);
-  for (int i = i0; i < i1; i++, o += plane) {
-    const bool iv = i + 1 < nx;
-    if (i + 1 < i1)
-      h_node_load(nxt, f, L, o + plane, (size_t)(i + 1) * ny + j, k, nz, plane, i + 2 < nx, jv,
-                  kv);
-    const float uyn = iv ? cur.uyn : 0.0f, uzn = iv ? cur.uzn : 0.0f;
-    const uint32_t m = CP ? mblk & cload(cp.pmask, 2 * (size_t)i) : 0u;
-    if (CP && m) {
-      float h0 = cur.ix, h1 = cur.iy, h2 = cur.iz;
-      if (jv && kv) h0 = h_expr<OE>(cur.da[0], h0, cur.db[0], cur.uz_j1, uzc, cur.uy_k1, uyc);
-      if (iv && kv) h1 = h_expr<OE>(cur.da[1], h1, cur.db[1], cur.ux_k1, cur.uxc, uzn, uzc);
-      if (iv && jv) h2 = h_expr<OE>(cur.da[2], h2, cur.db[2], uyn, uyc, cur.ux_j1, cur.uxc);
-      // T_p = u_other[node + e_p] - u_other[node] per (component, normal)
-      cpml_node<false, true>(cp.slabs, m, cp.par, true, i, j, k, cur.uz_j1 - uzc,
-                                    cur.uy_k1 - uyc, uzn - uzc, cur.ux_k1 - cur.uxc, uyn - uyc,
-                                    cur.ux_j1 - cur.uxc, cur.db[0], cur.db[1], cur.db[2], h0, h1,
-                                    h2);
-      ix[o] = h0, iy[o] = h1, iz[o] = h2;
-    } else {
-      if (jv && kv)  // curl_x = (uz[j+1] - uz[j]) - (uy[k+1] - uy[k])
-        ix[o] = h_expr<OE>(cur.da[0], cur.ix, cur.db[0], cur.uz_j1, uzc, cur.uy_k1, uyc);
-      if (iv && kv)  // curl_y = (ux[k+1] - ux[k]) - (uz[i+1] - uz[i])
-        iy[o] = h_expr<OE>(cur.da[1], cur.iy, cur.db[1], cur.ux_k1, cur.uxc, uzn, uzc);
-      if (iv && jv)  // curl_z = (uy[i+1] - uy[i]) - (ux[j+1] - ux[j])
-        iz[o] = h_expr<OE>(cur.da[2], cur.iz, cur.db[2], uyn, uyc, cur.ux_j1, cur.uxc);
-    }
-    uyc = uyn;
-    uzc = uzn;
-    cur = nxt;
+__global__ void __launch_bounds__(256, QW)
+    h_update_quad(Fields f, Lanes L, QuadGeom g, QuadCpml cp) {
+  int i, bx;
+  if (!quad_block(g, i, bx)) return;
+  int j, k0;
+  const bool in = quad_at(g, bx, j, k0);
+  bool fx = false, fy = false, fz = false;
+  if (CP) {
+    fx = quad_x_slab(cp, i);
+    quad_normals<false>(cp, g, in, i, j, k0, fy, fz);
   }
-}
-
-// What the E update of one node reads (kernel.rs:620-697).
-struct ENode {
-  float ix, iy, iz, iz_jm, iy_km, ix_km, ix_jm, ux, uy, uz;
-  float ca[3], cb[3];
-};
-
-__device__ __forceinline__ void e_node_load(ENode &q, const Fields &f, const Lanes &L, size_t o,
-                                            size_t r, int j, int k, int nz) {
-  const GAS float *ix = (const GAS float *)f.i[0], *iy = (const GAS float *)f.i[1];
-  const GAS float *iz = (const GAS float *)f.i[2];
-  const size_t oj = j > 0 ? o - nz : o, ok = k > 0 ? o - 1 : o;
-  q.ix = ix[o], q.iy = iy[o], q.iz = iz[o];
-  q.iz_jm = iz[oj], q.ix_jm = ix[oj], q.iy_km = iy[ok], q.ix_km = ix[ok];
-  q.ux = ((const GAS float *)f.u[0])[o], q.uy = ((const GAS float *)f.u[1])[o];
-  q.uz = ((const GAS float *)f.u[2])[o];
+  if (!in) return;
+  const int nz = g.nz, ny = g.ny, nx = g.nx;
+  const size_t plane = (size_t)ny * nz, ip = (size_t)i * plane, r = (size_t)i * ny + j;
+  const bool iv = i + 1 < nx, jv = j < ny - 1;
+  const size_t in1 = iv ? ip + plane : ip;
+  const unsigned vo = 4u * (unsigned)(j * nz + k0);
+  const unsigned vj = jv ? vo + 4u * (unsigned)nz : vo;
+  const unsigned ve = k0 + 4 < nz ? vo + 16u : vo;  // the node after the quad
+  f4 P[2];
+  if (CP && (fx || fy || fz)) quad_psi_first<false>(cp, g, fx, fy, i, j, k0, P);
+  const f4 ux = ld4(f.u[0] + ip, vo), uy = ld4(f.u[1] + ip, vo), uz = ld4(f.u[2] + ip, vo);
+  const float uxe = ld1(f.u[0] + ip, ve), uye = ld1(f.u[1] + ip, ve);
+  const f4 uxj = ld4(f.u[0] + ip, vj), uzj = ld4(f.u[2] + ip, vj);
+  f4 uyn = ld4(f.u[1] + in1, vo), uzn = ld4(f.u[2] + in1, vo);
+  f4 h[3], da[3], db[3];
 #pragma unroll
   for (int a = 0; a < 3; a++) {
-    q.ca[a] = coefg(L.l[a], r, k, nz, o);
-    q.cb[a] = coefg(L.l[3 + a], r, k, nz, o);
+    h[a] = ld4(f.i[a] + ip, vo);
+    da[a] = coef4(L.l[6 + a], ip, r, vo, k0, nz);
+    db[a] = coef4(L.l[9 + a], ip, r, vo, k0, nz);
   }
+  const f4 uxk = {ux[1], ux[2], ux[3], uxe}, uyk = {uy[1], uy[2], uy[3], uye};
+  if (!iv) uyn = uzn = f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    const bool kv = k0 + e < nz - 1;
+    // curl_x = (uz[j+1] - uz[j]) - (uy[k+1] - uy[k])
+    const float h0 = h_expr<OE>(da[0][e], h[0][e], db[0][e], uzj[e], uz[e], uyk[e], uy[e]);
+    // curl_y = (ux[k+1] - ux[k]) - (uz[i+1] - uz[i])
+    const float h1 = h_expr<OE>(da[1][e], h[1][e], db[1][e], uxk[e], ux[e], uzn[e], uz[e]);
+    // curl_z = (uy[i+1] - uy[i]) - (ux[j+1] - ux[j])
+    const float h2 = h_expr<OE>(da[2][e], h[2][e], db[2][e], uyn[e], uy[e], uxj[e], ux[e]);
+    h[0][e] = (jv && kv) ? h0 : h[0][e];
+    h[1][e] = (iv && kv) ? h1 : h[1][e];
+    h[2][e] = (iv && jv) ? h2 : h[2][e];
+  }
+  if (CP && (fx || fy || fz))  // T_p = u_other[node + e_p] - u_other[node]
+    quad_cpml<false>(cp, g, fx, fy, fz, i, j, k0, P, uzj - uz, uyk - uy, uzn - uz, uxk - ux,
+                     uyn - uy, uxj - ux, db, h);
+  const int ne = min(4, nz - k0);
+#pragma unroll
+  for (int a = 0; a < 3; a++) st_quad(f.i[a] + ip, vo, h[a], ne);
 }
 
 template <bool OE, bool CP>
-__global__ void __launch_bounds__(256) e_update_pf(Fields f, Lanes L, int nx, int ny, int nz,
-                                                   int chunk, CpmlIn cp) {
-  const int plane = ny * nz, gx = (plane + 255) / 256;
-  const int b = xcd_contiguous(blockIdx.x, gridDim.x);
-  const int p = (b % gx) * blockDim.x + threadIdx.x;
-  const uint32_t mblk =
-      CP ? block_slabs(cp.slabs, cp.nslab, (b % gx) * 256, min((b % gx) * 256 + 255, plane - 1), nz)
-         : 0u;
-  if (p >= plane) return;
-  const int j = p / nz, k = p - j * nz;
-  const int i0 = (b / gx) * chunk;
-  const int i1 = min(nx, i0 + chunk);
-  GAS float *ux = (GAS float *)f.u[0], *uy = (GAS float *)f.u[1], *uz = (GAS float *)f.u[2];
-  size_t o = (size_t)i0 * plane + p;
-  float iyp = i0 > 0 ? ((const GAS float *)f.i[1])[o - plane] : 0.0f;
-  float izp = i0 > 0 ? ((const GAS float *)f.i[2])[o - plane] : 0.0f;
-  ENode cur, nxt;
-  e_node_load(cur, f, L, o, (size_t)i0 * ny + j, j, k, nz);
-  for (int i = i0; i < i1; i++, o += plane) {
-    if (i + 1 < i1) e_node_load(nxt, f, L, o + plane, (size_t)(i + 1) * ny + j, j, k, nz);
-    const float hz_jm = j > 0 ? cur.iz_jm : 0.0f, hx_jm = j > 0 ? cur.ix_jm : 0.0f;
-    const float hy_km = k > 0 ? cur.iy_km : 0.0f, hx_km = k > 0 ? cur.ix_km : 0.0f;
-    const uint32_t m = CP ? mblk & cload(cp.pmask, 2 * (size_t)i + 1) : 0u;
-    if (CP && m) {
-      float e0 = cur.ux, e1 = cur.uy, e2 = cur.uz;
-      if (i + 1 < nx) e0 = e_expr<OE>(cur.ca[0], e0, cur.cb[0], cur.iz, hz_jm, cur.iy, hy_km);
-      if (j + 1 < ny) e1 = e_expr<OE>(cur.ca[1], e1, cur.cb[1], cur.ix, hx_km, cur.iz, izp);
-      if (k + 1 < nz) e2 = e_expr<OE>(cur.ca[2], e2, cur.cb[2], cur.iy, iyp, cur.ix, hx_jm);
-      // S_p = i_other[node] - i_other[node - e_p] (cpml.rs:495-521)
-      cpml_node<true, true>(cp.slabs, m, 0, true, i, j, k, cur.iz - hz_jm, cur.iy - hy_km,
-                                   cur.iz - izp, cur.ix - hx_km, cur.iy - iyp, cur.ix - hx_jm,
-                                   cur.cb[0], cur.cb[1], cur.cb[2], e0, e1, e2);
-      ux[o] = e0, uy[o] = e1, uz[o] = e2;
-    } else {
-      if (i + 1 < nx)  // curl_x = (iz[j] - iz[j-1]) - (iy[k] - iy[k-1])
-        ux[o] = e_expr<OE>(cur.ca[0], cur.ux, cur.cb[0], cur.iz, hz_jm, cur.iy, hy_km);
-      if (j + 1 < ny)  // curl_y = (ix[k] - ix[k-1]) - (iz[i] - iz[i-1])
-        uy[o] = e_expr<OE>(cur.ca[1], cur.uy, cur.cb[1], cur.ix, hx_km, cur.iz, izp);
-      if (k + 1 < nz)  // curl_z = (iy[i] - iy[i-1]) - (ix[j] - ix[j-1])
-        uz[o] = e_expr<OE>(cur.ca[2], cur.uz, cur.cb[2], cur.iy, iyp, cur.ix, hx_jm);
-    }
-    iyp = cur.iy;
-    izp = cur.iz;
-    cur = nxt;
+__global__ void __launch_bounds__(256, QW)
+    e_update_quad(Fields f, Lanes L, QuadGeom g, QuadCpml cp) {
+  int i, bx;
+  if (!quad_block(g, i, bx)) return;
+  int j, k0;
+  const bool in = quad_at(g, bx, j, k0);
+  bool fx = false, fy = false, fz = false;
+  if (CP) {
+    fx = quad_x_slab(cp, i);
+    quad_normals<true>(cp, g, in, i, j, k0, fy, fz);
   }
+  if (!in) return;
+  const int nz = g.nz, ny = g.ny, nx = g.nx;
+  const size_t plane = (size_t)ny * nz, ip = (size_t)i * plane, r = (size_t)i * ny + j;
+  const bool iv = i + 1 < nx, jv = j < ny - 1;
+  const size_t im1 = i > 0 ? ip - plane : ip;
+  const unsigned vo = 4u * (unsigned)(j * nz + k0);
+  const unsigned vj = j > 0 ? vo - 4u * (unsigned)nz : vo;
+  const unsigned ve = k0 > 0 ? vo - 4u : vo;  // the node before the quad
+  const f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  f4 P[2];
+  if (CP && (fx || fy || fz)) quad_psi_first<true>(cp, g, fx, fy, i, j, k0, P);
+  const f4 ix = ld4(f.i[0] + ip, vo), iy = ld4(f.i[1] + ip, vo), iz = ld4(f.i[2] + ip, vo);
+  float ixe = ld1(f.i[0] + ip, ve), iye = ld1(f.i[1] + ip, ve);
+  f4 ixj = ld4(f.i[0] + ip, vj), izj = ld4(f.i[2] + ip, vj);
+  f4 iyp = ld4(f.i[1] + im1, vo), izp = ld4(f.i[2] + im1, vo);
+  f4 u[3], ca[3], cb[3];
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    u[a] = ld4(f.u[a] + ip, vo);
+    ca[a] = coef4(L.l[a], ip, r, vo, k0, nz);
+    cb[a] = coef4(L.l[3 + a], ip, r, vo, k0, nz);
+  }
+  if (i == 0) iyp = izp = zero;
+  if (j == 0) ixj = izj = zero;
+  if (k0 == 0) ixe = iye = 0.0f;
+  const f4 ixk = {ixe, ix[0], ix[1], ix[2]}, iyk = {iye, iy[0], iy[1], iy[2]};
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    // curl_x = (iz[j] - iz[j-1]) - (iy[k] - iy[k-1])
+    const float e0 = e_expr<OE>(ca[0][e], u[0][e], cb[0][e], iz[e], izj[e], iy[e], iyk[e]);
+    // curl_y = (ix[k] - ix[k-1]) - (iz[i] - iz[i-1])
+    const float e1 = e_expr<OE>(ca[1][e], u[1][e], cb[1][e], ix[e], ixk[e], iz[e], izp[e]);
+    // curl_z = (iy[i] - iy[i-1]) - (ix[j] - ix[j-1])
+    const float e2 = e_expr<OE>(ca[2][e], u[2][e], cb[2][e], iy[e], iyp[e], ix[e], ixj[e]);
+    u[0][e] = iv ? e0 : u[0][e];
+    u[1][e] = jv ? e1 : u[1][e];
+    u[2][e] = k0 + e < nz - 1 ? e2 : u[2][e];
+  }
+  if (CP && (fx || fy || fz))  // S_p = i_other[node] - i_other[node - e_p] (cpml.rs:495-521)
+    quad_cpml<true>(cp, g, fx, fy, fz, i, j, k0, P, iz - izj, iy - iyk, iz - izp, ix - ixk,
+                    iy - iyp, ix - ixj, cb, u);
+  const int ne = min(4, nz - k0);
+#pragma unroll
+  for (int a = 0; a < 3; a++) st_quad(f.u[a] + ip, vo, u[a], ne);
 }
 
 // Loads/stores at a wave-uniform base plus a 32-bit per-lane byte offset,
@@ -3173,6 +3356,8 @@ struct ems_gpu {
   bool croff_wide = false;  // the pool is 4 GiB or more (only the tiled kernel addresses it)
   bool lanes_dirty = true;
   int par = 0;     // buffer holding the current state
+  int lock = 0;    // parity of the steps taken while the fused schedule was open (batches)
+  int boff = 0;    // during a batch run: par relative to the batch's
   Lane lanes[12]{};
   uint64_t lane_rows[12] = {0};
   std::vector<void *> lane_mem;
@@ -3193,9 +3378,12 @@ struct ems_gpu {
   bool ops_dirty = true, slabs_dirty = true;
   uint64_t step = 0;
   uint64_t *d_step = nullptr;
+  // until ems_gpu_set_schedule or a batch picks one, the schedule is the
+  // engine's choice (use_fused)
+  bool auto_sched = true;
   // fused schedule and its tiling
   bool fused = true, prefetch = true, rows = false, packed = false, band = false;
-  int unfused_pf = 11;  // ems_gpu_set_unfused_prefetch: bits 0, 1 load ahead; 2, 3 CPML in
+  int unfused_pf = 15;  // ems_gpu_set_unfused_prefetch: bits 0, 1 quads; 2, 3 CPML inside
   int xcd_group = 2;  // tile rows per XCD visit (2 measured best of 0, 1, 2, 4, 8)
   int tj = 7, nchunk = 0;
   // tile classes of the tiled step (ems_gpu_set_tile_classes): the tiles a
@@ -3231,15 +3419,13 @@ int fail(ems_gpu *h, int code, const std::string &m) {
     }                                                                                   \
   } while (0)
 
-int x_chunk(const ems_gpu *h, int *nchunks, bool pf) {
-  // Two planes per thread by default for the plain kernels: they are
-  // latency-bound, and more threads beat the reuse of a carried neighbour
-  // plane (measured on 385 x 385 x 257 nodes: 11 chunks 1.73 ms per step,
-  // 2-plane chunks 1.56 ms, 1-plane 1.57 ms). The kernels that load the
-  // next plane ahead march 8 planes (H on the same grid: 0.548 ms with
-  // 8-plane chunks, 0.565 ms with 32, 0.569 ms with 2; 0.647 ms plain). The
-  // schedule's x chunks, where set, take precedence.
-  int nch = h->nchunk > 0 ? h->nchunk : (pf ? (h->n[0] + 7) / 8 : (h->n[0] + 1) / 2);
+int x_chunk(const ems_gpu *h, int *nchunks) {
+  // Two planes per thread by default: the plain kernels are latency-bound,
+  // and more threads beat the reuse of a carried neighbour plane (measured
+  // on 385 x 385 x 257 nodes: 11 chunks 1.73 ms per step, 2-plane chunks
+  // 1.56 ms, 1-plane 1.57 ms). The schedule's x chunks, where set, take
+  // precedence.
+  int nch = h->nchunk > 0 ? h->nchunk : (h->n[0] + 1) / 2;
   if (nch < 1) nch = 1;
   if (nch > h->n[0]) nch = h->n[0];
   int chunk = (h->n[0] + nch - 1) / nch;
@@ -3269,9 +3455,6 @@ bool has_mid_ops(const ems_gpu *h) {
   return false;
 }
 
-// Whether steps run fused: not while an H source needs the serial gap
-// between the H and E updates (GAP_B, mod.rs:899-913; pool.rs:870-875).
-// The fused kernel keeps the slabs that reach a tile in a 32-bit mask.
 bool has_magnetic_poles(const ems_gpu *h) {
   for (auto &o : h->ops)
     if (o.type == OP_POLES && o.side[1].n > 0) return true;
@@ -3299,11 +3482,29 @@ bool has_upml(const ems_gpu *h) {
   return false;
 }
 
-bool use_fused(const ems_gpu *h) {
+// Whether steps can run fused: not while an H source needs the serial gap
+// between the H and E updates (GAP_B, mod.rs:899-913; pool.rs:870-875).
+// The fused kernel keeps the slabs that reach a tile in a 32-bit mask.
+bool fused_eligible(const ems_gpu *h) {
   size_t ns = 0;
   for (auto &s : h->slabs) ns += s.len != 0;
   return h->fused && !has_hsrc(h) && !has_magnetic_poles(h) && !has_gap_kernels(h) &&
          !has_upml(h) && ns <= 32;
+}
+
+// Whether the quad kernels take this grid: a plane's byte offsets in 32
+// bits.
+bool quad_ok(const ems_gpu *h) { return h->plane < ((size_t)1 << 29); }
+
+// An engine whose schedule nobody set steps unfused: the quad kernels read
+// and write each node twice a step instead of once, but at the copy rate,
+// without halo rows or a march along x, and with the CPML inside: 13.7
+// against 47 us per step on 25^3 nodes (the fused default, one block
+// marching 25 planes), 41 against 74 (132 x 98 x 75 nodes with CPML, the
+// best fused tiling), 2.60 against 2.83 ms (513^3, the best fused tiling;
+// the fused default 4.3).
+bool use_fused(const ems_gpu *h) {
+  return !(h->auto_sched && quad_ok(h)) && fused_eligible(h);
 }
 
 // The dispersive media as slab hooks (dispersive.rs:1700-1750), in
@@ -3337,54 +3538,118 @@ int launch_poles(ems_gpu *h, int stage, const Fields &f, const Fields &fp, bool 
   return 0;
 }
 
-// Whether side `side` (0 H, 1 E) corrects its CPML slabs inside its
-// unfused update: bit 2 + side of the unfused switch with the side's
-// loading-ahead kernel (bit side), and the slab table built for it (every slab but the z-normal
-// suffix, whose columns would run the slab code in a few lanes of most
-// waves; those keep their launches, after the kernel, so the corrections
-// of a node keep the registration order; at most 32 for the planes'
-// masks).
-bool cpml_folded(const ems_gpu *h, int side) {
-  if (use_fused(h) || !(h->unfused_pf & (4 << side)) || !(h->unfused_pf & (1 << side)) ||
-      !h->d_fslabs || !h->d_pmask || h->split_state != 2)
-    return false;
-  int n = 0;
-  for (auto &s : h->slabs) n += s.len != 0 && !s.out;
-  return n > 0 && n <= 32;
+// The CPML slabs of a side in the form the quad kernels correct them
+// (QuadCpml; H psi of buffer par). False where that form does not hold them
+// all: a component's slabs of its first normal after those of its second,
+// more than one slab per end, boxes that do not span the component, or two
+// ends that meet in one quad.
+bool quad_cpml_args(const ems_gpu *h, int side, int par, QuadCpml *out) {
+  QuadCpml cp;
+  for (auto &c : cp.e)
+    for (auto &n : c)
+      for (auto &e : n) e = CpmlEnd{nullptr, nullptr, INT32_MAX / 2, 0};
+  for (auto &s : h->slabs) {
+    const SlabArg &a = s.arg;
+    if (s.len == 0 || a.e_side != side) continue;
+    for (int d = 0; d < 3; d++)
+      if (d != a.normal) {
+        // E edges of a component end one short of the last line along it,
+        // dual edges along the other two directions
+        const int ext = h->n[d] - ((a.e_side != 0) == (d == a.comp) ? 1 : 0);
+        if (a.lo[d] != 0 || a.hi[d] != ext) return false;
+      }
+    const int w = pair_of(a.comp, a.normal);
+    CpmlEnd &lo = cp.e[a.comp][w][0], &hi = cp.e[a.comp][w][1];
+    if (w == 0)  // (the second normal's corrections follow the first's)
+      for (auto &e : cp.e[a.comp][1])
+        if (e.psi) return false;
+    CpmlEnd in{s.d_psi[side ? 0 : par], s.d_b, a.lo[a.normal], a.hi[a.normal]};
+    if (!lo.psi) {
+      lo = in;
+    } else if (!hi.psi) {
+      hi = in;
+      if (hi.lo < lo.lo) std::swap(lo, hi);
+      const int gap = a.normal == 2 ? hi.lo / 4 * 4 : hi.lo;  // (whole quads along z)
+      if (gap < lo.hi) return false;
+    } else {
+      return false;
+    }
+  }
+  // a lone slab is the low end; the absent high end starts past the grid
+  *out = cp;
+  return true;
 }
 
-int n_fslabs(const ems_gpu *h);
+// Whether side `side` (0 H, 1 E) corrects its CPML slabs inside its
+// unfused update: bit 2 + side of the unfused switch with the side's quad
+// kernel (bit side).
+bool cpml_folded(const ems_gpu *h, int side, QuadCpml *cp = nullptr) {
+  if (use_fused(h) || !quad_ok(h) || !(h->unfused_pf & (4 << side)) ||
+      !(h->unfused_pf & (1 << side)))
+    return false;
+  bool any = false;
+  for (auto &s : h->slabs) any = any || (s.len != 0 && s.arg.e_side == side);
+  QuadCpml tmp;
+  return any && quad_cpml_args(h, side, h->par, cp ? cp : &tmp);
+}
 
-#define UNFUSED_LAUNCH(K, grid_, cp_on)                                                   \
-  do {                                                                                    \
-    if (h->oe) {                                                                          \
-      if (cp_on)                                                                          \
-        hipLaunchKernelGGL((K<true, true>), grid_, dim3(256), 0, h->stream, f, lanes_arg(h), \
-                           h->n[0], h->n[1], h->n[2], chunk, cp);                         \
-      else                                                                                \
-        hipLaunchKernelGGL((K<true, false>), grid_, dim3(256), 0, h->stream, f, lanes_arg(h), \
-                           h->n[0], h->n[1], h->n[2], chunk, cp);                         \
-    } else {                                                                              \
-      if (cp_on)                                                                          \
-        hipLaunchKernelGGL((K<false, true>), grid_, dim3(256), 0, h->stream, f, lanes_arg(h), \
-                           h->n[0], h->n[1], h->n[2], chunk, cp);                         \
-      else                                                                                \
-        hipLaunchKernelGGL((K<false, false>), grid_, dim3(256), 0, h->stream, f,           \
-                           lanes_arg(h), h->n[0], h->n[1], h->n[2], chunk, cp);           \
-    }                                                                                     \
+// The quad kernels' geometry and grid.
+QuadGeom quad_geom(const ems_gpu *h, int side, bool cpf, unsigned *blocks) {
+  QuadGeom g;
+  g.nx = h->n[0], g.ny = h->n[1], g.nz = h->n[2];
+  const int nq = (g.nz + 3) / 4;
+  // the first and last quads that a z-normal slab of the side reaches
+  g.ql = g.qh = 0;
+  if (cpf)
+    for (auto &s : h->slabs) {
+      if (s.len == 0 || s.arg.e_side != side || s.arg.normal != 2) continue;
+      if (s.arg.lo[2] < g.nz - s.arg.hi[2]) g.ql = std::max(g.ql, (s.arg.hi[2] + 3) / 4);
+      else g.qh = std::max(g.qh, nq - s.arg.lo[2] / 4);
+    }
+  if (g.ql + g.qh >= nq) g.ql = g.qh = 0;
+  g.nm = nq - g.ql - g.qh;
+  g.gm = (int)(((size_t)g.ny * g.nm + 255) / 256);
+  g.gx = g.gm + (int)(((size_t)g.ny * (g.ql + g.qh) + 255) / 256);
+  // Grids whose fields stay in the 256 MB of cache behind the L2s: each XCD
+  // one contiguous eighth of the grid, so that a block's neighbours in j and
+  // x ran on its own L2 (97 x 74-node planes, 131 of them: 40.8 us per step
+  // against 43.5 in runs of 24 and 55.7 in plain order). Larger grids: runs
+  // of 24 blocks (some 48 rows of 513 nodes), since eight far-apart regions
+  // read from memory at once cost more than the sharing gains (513^3 nodes:
+  // 2.60 ms per step, 2.65 in plain order, 2.86 in contiguous eighths).
+  const unsigned n = (unsigned)g.gx * (unsigned)g.nx;
+  const bool cached = h->N * 24 <= ((size_t)256 << 20);
+  g.run = cached ? (int)((n + 7) / 8) : 24;
+  const unsigned w = 8u * (unsigned)g.run;
+  *blocks = (n + w - 1) / w * w;
+  return g;
+}
+
+#define QUAD_LAUNCH(K)                                                                          \
+  do {                                                                                          \
+    if (h->oe && cpf)                                                                           \
+      hipLaunchKernelGGL((K<true, true>), dim3(nb), dim3(256), 0, h->stream, f, lanes_arg(h), g, cp); \
+    else if (h->oe)                                                                             \
+      hipLaunchKernelGGL((K<true, false>), dim3(nb), dim3(256), 0, h->stream, f, lanes_arg(h), g, cp); \
+    else if (cpf)                                                                               \
+      hipLaunchKernelGGL((K<false, true>), dim3(nb), dim3(256), 0, h->stream, f, lanes_arg(h), g, cp); \
+    else                                                                                        \
+      hipLaunchKernelGGL((K<false, false>), dim3(nb), dim3(256), 0, h->stream, f, lanes_arg(h), g, cp); \
   } while (0)
 
 int launch_h(ems_gpu *h, const Fields &f) {
-  int nch, chunk = x_chunk(h, &nch, (h->unfused_pf & 1) != 0);
+  if ((h->unfused_pf & 1) && quad_ok(h)) {
+    unsigned nb;
+    QuadCpml cp{};
+    const bool cpf = cpml_folded(h, 0, &cp);
+    const QuadGeom g = quad_geom(h, 0, cpf, &nb);
+    QUAD_LAUNCH(h_update_quad);
+    CK(h, hipGetLastError());
+    return 0;
+  }
+  int nch, chunk = x_chunk(h, &nch);
   dim3 grid((unsigned)((h->plane + 255) / 256), (unsigned)nch);
-  // the loading-ahead kernel runs one-dimensional (see xcd_contiguous; the
-  // two-plane kernel measured slower so: E 0.526 against 0.503 ms)
-  const dim3 line(grid.x * grid.y);
-  if (h->unfused_pf & 1) {
-    const bool cpf = cpml_folded(h, 0);
-    const CpmlIn cp{h->d_fslabs, h->d_pmask, cpf ? n_fslabs(h) : 0, h->par};
-    UNFUSED_LAUNCH(h_update_pf, line, cpf);
-  } else if (h->oe)
+  if (h->oe)
     hipLaunchKernelGGL(h_update<true>, grid, dim3(256), 0, h->stream, f, lanes_arg(h), h->n[0],
                        h->n[1], h->n[2], chunk);
   else
@@ -3395,14 +3660,18 @@ int launch_h(ems_gpu *h, const Fields &f) {
 }
 
 int launch_e(ems_gpu *h, const Fields &f) {
-  int nch, chunk = x_chunk(h, &nch, (h->unfused_pf & 2) != 0);
+  if ((h->unfused_pf & 2) && quad_ok(h)) {
+    unsigned nb;
+    QuadCpml cp{};
+    const bool cpf = cpml_folded(h, 1, &cp);
+    const QuadGeom g = quad_geom(h, 1, cpf, &nb);
+    QUAD_LAUNCH(e_update_quad);
+    CK(h, hipGetLastError());
+    return 0;
+  }
+  int nch, chunk = x_chunk(h, &nch);
   dim3 grid((unsigned)((h->plane + 255) / 256), (unsigned)nch);
-  const dim3 line(grid.x * grid.y);
-  if (h->unfused_pf & 2) {
-    const bool cpf = cpml_folded(h, 1);
-    const CpmlIn cp{h->d_fslabs, h->d_pmask, cpf ? n_fslabs(h) : 0, 0};
-    UNFUSED_LAUNCH(e_update_pf, line, cpf);
-  } else if (h->oe)
+  if (h->oe)
     hipLaunchKernelGGL(e_update<true>, grid, dim3(256), 0, h->stream, f, lanes_arg(h), h->n[0],
                        h->n[1], h->n[2], chunk);
   else
@@ -3411,12 +3680,12 @@ int launch_e(ems_gpu *h, const Fields &f) {
   CK(h, hipGetLastError());
   return 0;
 }
-#undef UNFUSED_LAUNCH
+#undef QUAD_LAUNCH
 
 int launch_cpml(ems_gpu *h, const Fields &f, int e_side, int par) {
-  const bool folded = cpml_folded(h, e_side);  // then only the suffix runs here
+  const bool folded = cpml_folded(h, e_side);
   for (auto &s : h->slabs) {
-    if (s.arg.e_side != e_side || s.len == 0 || (folded && !s.out)) continue;
+    if (s.arg.e_side != e_side || s.len == 0 || folded) continue;
     const Lane cf = h->lanes[e_side ? 3 + s.arg.comp : 9 + s.arg.comp];
     SlabArg a = s.arg;
     a.psi = e_side ? s.d_psi[0] : s.d_psi[par];
@@ -3532,22 +3801,12 @@ int upload_out_slabs(ems_gpu *h) {
 }
 
 // state: 0 every slab in the table; 1 the fused kernel's split (the
-// z-normal suffix corrected by its passes outside it); 2 the same suffix
-// left to the unfused schedule's own slab launches (no outside tables).
+// z-normal suffix corrected by its passes outside it).
 int upload_fslabs(ems_gpu *h, int state) {
   if (!h->slabs_dirty && h->split_state == state) return 0;
   mark_out_slabs(h, state != 0);
-  int rc = state == 2 ? 0 : upload_out_slabs(h);
+  int rc = upload_out_slabs(h);
   if (rc) return rc;
-  if (state == 2) {
-    if (h->d_hout) CK(h, hipFree(h->d_hout));
-    if (h->d_eout) CK(h, hipFree(h->d_eout));
-    if (h->d_pmask_o) CK(h, hipFree(h->d_pmask_o));
-    h->d_hout = h->d_eout = nullptr;
-    h->d_pmask_o = nullptr;
-    h->n_hout = h->n_eout = 0;
-    h->hout_total = h->eout_total = 0;
-  }
   h->split_state = state;
   h->slab_gen++;
   if (h->d_fslabs) CK(h, hipFree(h->d_fslabs));
@@ -4097,7 +4356,7 @@ int build_pool(ems_gpu *h) {
       total += h->lane_rows[l] * (uint64_t)nz;
     }
   float *pool = nullptr;
-  CK(h, hipMalloc(&pool, total * sizeof(float)));
+  CK(h, hipMalloc(&pool, (total + QUAD_PAD) * sizeof(float)));
   CK(h, hipMemset(pool, 0, (size_t)nz * sizeof(float)));
   for (int l = 0; l < 12; l++)
     if (h->lanes[l].rows)
@@ -4268,11 +4527,7 @@ int prepare(ems_gpu *h, uint64_t steps, bool allow_split = true) {
     }
   }
   if (grown) h->ops_dirty = true;
-  // the fused kernel's split, or the unfused kernels' CPML fold (bits 2, 3
-  // of the unfused switch), which takes the slabs but the z-normal suffix
-  const int split = (allow_split && h->cpml_split && tiled_fused(h))
-                        ? 1
-                        : ((!use_fused(h) && ((h->unfused_pf >> 2) & h->unfused_pf & 3)) ? 2 : 0);
+  const int split = (allow_split && h->cpml_split && tiled_fused(h)) ? 1 : 0;
   if (h->slabs_dirty || h->split_state != split) {
     drop_graphs(h);
     int rc = upload_fslabs(h, split);
@@ -4339,6 +4594,7 @@ void advance_counts(ems_gpu *h, uint64_t steps) {
     o.count += (b + o.interval - 1) / o.interval - (a + o.interval - 1) / o.interval;
   }
   h->step += steps;
+  if (fused_eligible(h)) h->lock ^= (int)(steps & 1);
 }
 
 // Scratch of one evaluation, in doubles: a sum per H row (nx * (3 ny - 2)),
@@ -4472,6 +4728,17 @@ int run_steps(ems_gpu *h, uint64_t n) {
   return 0;
 }
 
+// A device array of n floats (src, or zeros) between QUAD_PAD floats of
+// padding, which quad accesses at the ends of a slab's rows may read.
+int upload_padded(ems_gpu *h, float **dst, const float *src, size_t n) {
+  float *p = nullptr;
+  CK(h, hipMalloc(&p, (n + 2 * QUAD_PAD) * sizeof(float)));
+  *dst = p + QUAD_PAD;
+  CK(h, hipMemset(p, 0, (n + 2 * QUAD_PAD) * sizeof(float)));
+  if (src && n) CK(h, hipMemcpy(*dst, src, n * sizeof(float), hipMemcpyHostToDevice));
+  return 0;
+}
+
 int upload(ems_gpu *h, void **dst, const void *src, size_t bytes) {
   CK(h, hipMalloc(dst, bytes ? bytes : 1));
   if (bytes) CK(h, hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice));
@@ -4514,7 +4781,7 @@ int ems_gpu_create(const ems_grid_desc *d, ems_gpu **out) {
   auto init = [&]() -> int {
     CK(h, hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
     for (int b = 0; b < 2; b++) {
-      CK(h, hipMalloc(&h->fbuf[b], 6 * N * sizeof(float)));
+      CK(h, hipMalloc(&h->fbuf[b], (6 * N + QUAD_PAD) * sizeof(float)));
       CK(h, hipMemset(h->fbuf[b], 0, 6 * N * sizeof(float)));
       for (int a = 0; a < 3; a++) {
         h->fb[b].u[a] = h->fbuf[b] + a * N;
@@ -4545,9 +4812,8 @@ void ems_gpu_destroy(ems_gpu *h) {
   if (h->cpool) (void)hipFree(h->cpool);
   if (h->croff) (void)hipFree(h->croff);
   for (auto &s : h->slabs) {
-    (void)hipFree(s.d_b), (void)hipFree(s.d_a), (void)hipFree(s.d_k);
-    (void)hipFree(s.d_psi[0]);
-    if (s.d_psi[1]) (void)hipFree(s.d_psi[1]);
+    for (float *q : {s.d_b, s.d_psi[0], s.d_psi[1]})
+      if (q) (void)hipFree(q - QUAD_PAD);
     if (s.d_delta) (void)hipFree(s.d_delta);
   }
   if (h->d_fslabs) (void)hipFree(h->d_fslabs);
@@ -4653,15 +4919,20 @@ int ems_gpu_add_cpml(ems_gpu *h, const ems_cpml_slab *s, int n) {
     for (int d = 0; d < 3; d++) a.lo[d] = in.lo[d], a.hi[d] = in.hi[d];
     const int depth = in.hi[in.normal] - in.lo[in.normal];
     int rc;
-    if ((rc = upload(h, (void **)&hs.d_b, in.b, depth * sizeof(float)))) return rc;
-    if ((rc = upload(h, (void **)&hs.d_a, in.a, depth * sizeof(float)))) return rc;
-    if ((rc = upload(h, (void **)&hs.d_k, in.k, depth * sizeof(float)))) return rc;
-    hs.len = (size_t)(in.hi[0] - in.lo[0]) * (in.hi[1] - in.lo[1]) * (in.hi[2] - in.lo[2]);
-    const size_t bytes = (hs.len ? hs.len : 1) * sizeof(float);
-    for (int b = 0; b < (a.e_side ? 1 : 2); b++) {
-      CK(h, hipMalloc(&hs.d_psi[b], bytes));
-      CK(h, hipMemset(hs.d_psi[b], 0, bytes));
+    // b, a and k by depth, each with QUAD_PAD floats of padding before and
+    // after it, one behind the other
+    const size_t seg = (size_t)depth + 2 * QUAD_PAD;
+    std::vector<float> bak(3 * seg, 0.0f);
+    for (int d = 0; d < depth; d++) {
+      bak[QUAD_PAD + d] = in.b[d];
+      bak[seg + QUAD_PAD + d] = in.a[d];
+      bak[2 * seg + QUAD_PAD + d] = in.k[d];
     }
+    if ((rc = upload_padded(h, &hs.d_b, bak.data() + QUAD_PAD, 3 * seg - 2 * QUAD_PAD))) return rc;
+    hs.d_a = hs.d_b + seg, hs.d_k = hs.d_a + seg;
+    hs.len = (size_t)(in.hi[0] - in.lo[0]) * (in.hi[1] - in.lo[1]) * (in.hi[2] - in.lo[2]);
+    for (int b = 0; b < (a.e_side ? 1 : 2); b++)
+      if ((rc = upload_padded(h, &hs.d_psi[b], nullptr, hs.len))) return rc;
     a.b = hs.d_b, a.a = hs.d_a, a.k = hs.d_k, a.psi = nullptr;
     h->slabs.push_back(hs);
   }
@@ -5552,6 +5823,7 @@ int ems_gpu_set_schedule(ems_gpu *h, int fused, int tile_rows, int x_chunks) {
   h->band = fused == 6;
   if (x_chunks < 0) return fail(h, EMS_E_INVALID, "x_chunks must be >= 0");
   h->fused = fused != 0;
+  h->auto_sched = false;
   if (tile_rows) h->tj = tile_rows;
   h->nchunk = x_chunks;
   drop_graphs(h);
@@ -6247,6 +6519,7 @@ struct ems_gpu_batch {
   int tj = 7, nchunk = 0, oe = 0;
   bool prefetch = true, packed = false;
   std::vector<int> active;        // the set the graphs were captured for
+  std::vector<int> boffs;         // their buffer parities relative to the first one
   FusedArgs *d_args[2] = {nullptr, nullptr};
   GapArgs *d_gap[2] = {nullptr, nullptr};
   uint32_t *d_seg = nullptr;
@@ -6302,14 +6575,15 @@ int batch_args(ems_gpu_batch *b, const std::vector<int> &act) {
       ems_gpu *h = b->m[act[q]];
       const FusedGeom g = b->packed ? packed_geom(h, b->nchunk) : fused_geom(h);
       FusedArgs &a = fa[q];
-      a.A = h->fbuf[p], a.B = h->fbuf[1 - p], a.N = h->N;
+      const int hp = p ^ h->boff;  // the model's own parity
+      a.A = h->fbuf[hp], a.B = h->fbuf[1 - hp], a.N = h->N;
       a.cpool = h->cpool, a.croff = (const uint32_t *)h->croff, a.slabs = h->d_fslabs,
       a.pmask = h->d_pmask;
-      a.nslab = n_fslabs(h), a.par = p, a.nx = h->n[0], a.ny = h->n[1], a.nz = h->n[2];
+      a.nslab = n_fslabs(h), a.par = hp, a.nx = h->n[0], a.ny = h->n[1], a.nz = h->n[2];
       a.tk = g.tk, a.chunk = g.chunk, a.ktiles = g.ktiles, a.jtiles = g.jtiles, a.ntiles = g.ntiles;
       if (p == 0) seg[q + 1] = seg[q] + (uint32_t)g.nblocks;
       GapArgs &gg = ga[q];
-      gg.f = h->fb[1 - p], gg.fp = h->fb[p], gg.ops = h->d_ops, gg.nops = (int)h->ops.size();
+      gg.f = h->fb[1 - hp], gg.fp = h->fb[hp], gg.ops = h->d_ops, gg.nops = (int)h->ops.size();
       gg.step = h->d_step;
     }
     BCK(b, hipMemcpy(b->d_args[p], fa.data(), n * sizeof(FusedArgs), hipMemcpyHostToDevice));
@@ -6363,7 +6637,8 @@ int batch_enqueue_step(ems_gpu_batch *b, const std::vector<int> &act, int par) {
     ems_gpu *h = b->m[q];
     const hipStream_t own = h->stream;
     h->stream = b->stream;
-    const int rc = launch_poles(h, 1, h->fb[par ^ 1], h->fb[par], true);
+    const int hp = par ^ h->boff;
+    const int rc = launch_poles(h, 1, h->fb[hp ^ 1], h->fb[hp], true);
     h->stream = own;
     if (rc) return bfail(b, rc, h->err);
   }
@@ -6466,10 +6741,13 @@ int ems_gpu_batch_run(ems_gpu_batch *b, const uint8_t *active, uint64_t n) {
   for (size_t q = 0; q < b->m.size(); q++)
     if (!active || active[q]) act.push_back((int)q);
   if (act.empty() || n == 0) return EMS_OK;
-  const int par = b->m[act[0]]->par;
+  const int par = b->m[act[0]]->par, lock = b->m[act[0]]->lock;
+  std::vector<int> boffs;
   for (int q : act) {
     ems_gpu *h = b->m[q];
     if (h->dead) return bfail(b, EMS_E_DEVICE, "model " + std::to_string(q) + ": " + h->err);
+    if (h->auto_sched || !h->fused) drop_graphs(h);  // (captured for the unfused schedule)
+    h->auto_sched = false;
     h->fused = true, h->rows = false, h->band = false, h->prefetch = b->prefetch, h->tj = b->tj;
     h->packed = b->packed;
     h->nchunk = b->nchunk;
@@ -6482,7 +6760,9 @@ int ems_gpu_batch_run(ems_gpu_batch *b, const uint8_t *active, uint64_t n) {
                    "model " + std::to_string(q) +
                        " needs the unfused schedule (H source, magnetic poles, plane wave, "
                        "cut-face currents, openEMS PML layers or more than 32 CPML slabs)");
-    if (h->par != par) return bfail(b, EMS_E_INVALID, "models of a batch step in lockstep");
+    if (h->lock != lock) return bfail(b, EMS_E_INVALID, "models of a batch step in lockstep");
+    h->boff = h->par ^ par;
+    boffs.push_back(h->boff);
     const int rc = prepare(h, n, false);
     if (rc) return bfail(b, rc, h->err);
     if (h->croff_wide)
@@ -6490,6 +6770,8 @@ int ems_gpu_batch_run(ems_gpu_batch *b, const uint8_t *active, uint64_t n) {
                    "model " + std::to_string(q) + " has a coefficient pool of 4 GiB or more");
     BCK(b, hipStreamSynchronize(h->stream));
   }
+  if (boffs != b->boffs) batch_drop_graphs(b);  // (they hold the models' buffers)
+  b->boffs = boffs;
   int rc = batch_args(b, act);
   if (rc) return rc;
   if (!b->graphs) {  // the same launches, queued one by one
@@ -6499,7 +6781,7 @@ int ems_gpu_batch_run(ems_gpu_batch *b, const uint8_t *active, uint64_t n) {
     BCK(b, hipStreamSynchronize(b->stream));
     for (int q : act) {
       ems_gpu *h = b->m[q];
-      h->par = p;
+      h->par = p ^ h->boff;
       advance_counts(h, n);
     }
     return EMS_OK;
@@ -6526,7 +6808,7 @@ int ems_gpu_batch_run(ems_gpu_batch *b, const uint8_t *active, uint64_t n) {
   BCK(b, hipStreamSynchronize(b->stream));
   for (int q : act) {
     ems_gpu *h = b->m[q];
-    h->par = p;
+    h->par = p ^ h->boff;
     advance_counts(h, n);
   }
   return EMS_OK;

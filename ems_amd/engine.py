@@ -753,7 +753,7 @@ class Engine:
         self._dense_lanes = lanes
         self._owns_lanes = False
         self._pool = pool
-        self.unfused_prefetch = 11
+        self.unfused_prefetch = 15
         self.setup: List[tuple] = []
         self.ops: list = []
         self._tables: list = []
@@ -1116,11 +1116,11 @@ class Engine:
         self._check(nat.ems_gpu_set_tile_classes(self._h, 1 if on else 0))
 
     def set_unfused_prefetch(self, which: int = 11) -> None:
-        """The unfused kernels: bits 0 (H) and 1 (E) march longer x chunks
-        with the next plane's inputs loaded ahead; bits 2 (H) and 3 (E),
-        with the side's loading-ahead kernel, correct the side's CPML slabs
-        (but a z-normal suffix) inside it. Default 11; the same values
-        either way."""
+        """The unfused kernels: bits 0 (H) and 1 (E) take four nodes of a z
+        row per thread (else one node, two x-planes); bits 2 (H) and 3 (E),
+        with the side's bit 0 or 1, correct the side's CPML slabs inside the
+        update instead of in launches of their own. An engine starts with
+        all four; the same values either way."""
         self._check(nat.ems_gpu_set_unfused_prefetch(self._h, int(which)))
         self.unfused_prefetch = int(which)
 
@@ -1130,28 +1130,29 @@ class Engine:
         self._check(nat.ems_gpu_set_xcd_group(self._h, int(group)))
 
     def autotune(self, candidates=None, steps_each: int = 4, xcd_groups=(1, 2, 4, 8)):
-        """Times a few real steps of each fused tiling on this engine (they
+        """Times a few real steps of each schedule on this engine (they
         advance the simulation like any other steps) and keeps the fastest.
-        Candidates are (mode, tile_rows, x_chunks), mode 1 with and 2
-        without the next-plane prefetch (mode 3, the full-row kernel, only
-        when listed). Returns the choice with its mean kernel time in ms,
+        Candidates are (mode, tile_rows, x_chunks), mode 0 unfused, mode 1
+        with and 2 without the next-plane prefetch (mode 3, the full-row
+        kernel, only when listed). Returns the choice with its mean kernel time in ms,
         and all timings."""
         if candidates is None:
-            candidates = [(m, t, c) for m in (1, 2) for t in (3, 7, 15)
-                          for c in (0, 16, 32, 64, 96, 128)]
+            candidates = [(0, 0, 0)]
+            candidates += [(m, t, c) for m in (1, 2) for t in (3, 7, 15)
+                           for c in (0, 16, 32, 64, 96, 128)]
             if self.grid.nodes()[2] <= 64:
                 candidates += [(m, 7, c) for m in (4, 5) for c in (0, 16, 32, 64)]
         results = []
         for m, t, c in candidates:
             self.set_schedule(m, t, c)
             self.time_kernels(1)  # first launch of a tiling: not timed
-            ms = self.time_kernels(steps_each)[0]
+            ms = sum(self.time_kernels(steps_each)[:2])
             results.append((m, t, c, ms))
         best = min(results, key=lambda r: r[3])
         self.set_schedule(best[0], best[1], best[2])
         # then the XCD grouping of the tile order for that tiling
         groups = []
-        for g in xcd_groups:
+        for g in xcd_groups if best[0] else ():
             self.set_xcd_group(g)
             self.time_kernels(1)
             groups.append((g, self.time_kernels(steps_each)[0]))

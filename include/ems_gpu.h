@@ -460,8 +460,8 @@ double ems_gpu_dt(const ems_gpu *h);
  * the full-row variant: one wave per row, nz <= 576, tile_rows 3 or 7;
  * 4 packed short rows: 64 / nz whole k-rows per wave, nz <= 64, else the
  * tiled kernel; 5 the same without the prefetch); tile_rows 3, 7 or 15
- * (0 keeps the current);
- * x_chunks 0 = automatic. Steps that need the serial gap between the H and
+ * (0 keeps the current); x_chunks 0 = automatic. Until this is called the
+ * engine steps unfused (measured fastest at every size). Steps that need the serial gap between the H and
  * E updates (H sources) always run unfused. */
 int ems_gpu_set_schedule(ems_gpu *h, int fused, int tile_rows, int x_chunks);
 
@@ -477,14 +477,13 @@ int ems_gpu_set_cpml_split(ems_gpu *h, int on);
  * code (fewer registers, more waves per SIMD). Same results either way. */
 int ems_gpu_set_tile_classes(ems_gpu *h, int on);
 /* The unfused H and E kernels (no reference counterpart). `which` bit 0
- * (H) and bit 1 (E): the side's threads march a chunk of x-planes (8 by
- * default; the schedule's x chunks where set) with the next plane's inputs
- * loaded before the present plane is computed, else two planes without
- * that. Bit 2 (H) and bit 3 (E), with the side's bit 0 or 1: the side's
- * CPML slabs, but a suffix of z-normal ones, are corrected inside the
- * update instead of in launches of their own. Default 11 (H and E load
- * ahead, E corrects its slabs inside: measured fastest). Same results
- * either way; 0 to 15, else EMS_E_INVALID. */
+ * (H) and bit 1 (E): the side's threads take four consecutive nodes of a z
+ * row each, else one node of two x-planes. Bit 2 (H) and bit 3 (E), with
+ * the side's bit 0 or 1: the side's CPML slabs are corrected inside the
+ * update instead of in launches of their own (where each component's slabs
+ * span it and come in the order of their normals). An engine starts with
+ * 15 (measured fastest). Same results either way; 0 to 15, else
+ * EMS_E_INVALID. */
 int ems_gpu_set_unfused_prefetch(ems_gpu *h, int which);
 
 /* Tile order of the fused kernels (no reference counterpart): groups of

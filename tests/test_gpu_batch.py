@@ -124,3 +124,24 @@ def test_batch_refuses_models_out_of_step_and_duplicates():
         E.EngineBatch([a, a])
     a.close()
     b.close()
+
+
+def test_batch_after_single_runs():
+    """Models that stepped on their own first, one of them on another
+    schedule (the same steps taken, the state in another buffer), step on
+    together like engines of their own."""
+    ms = models()[:2]
+    (a, _), (b, _), (c, _), (d, _) = (engine(ms[q]) for q in (0, 1, 0, 1))
+    b.set_schedule(1, 3, 2)
+    a.run(3)
+    b.run(3)
+    batch = E.EngineBatch([a, b])
+    for n in (2, 21):
+        batch.run(n)
+    a.run(2)  # (on the schedule the batch left it on)
+    c.run(28)
+    d.run(26)
+    for x, y in ((a, c), (b, d)):
+        for f in (0, 1):
+            for k in range(3):
+                assert np.array_equal(x._read(f, k).view(np.uint32), y._read(f, k).view(np.uint32))
