@@ -587,16 +587,13 @@ struct QuadGeom {
   int run;    // consecutive blocks an XCD takes at a time
 };
 
-// Plane and in-plane block of this block. Blocks go round-robin to the 8
-// XCDs; each XCD takes `run` consecutive blocks of the grid at a time.
-__device__ __forceinline__ bool quad_block(const QuadGeom &g, int &i, int &bx) {
-  unsigned b = blockIdx.x;
-  const unsigned w = 8u * (unsigned)g.run, q = b % w;
-  b = b - q + (q % 8u) * (unsigned)g.run + q / 8u;
-  i = (int)(b / (unsigned)g.gx);
-  bx = (int)(b - (unsigned)i * (unsigned)g.gx);
-  return i < g.nx;
+// Blocks go round-robin to the 8 XCDs; each XCD takes `run` consecutive
+// places of the grid at a time (a bijection of every 8 run blocks).
+__device__ __forceinline__ unsigned quad_order(unsigned b, int run) {
+  const unsigned w = 8u * (unsigned)run, q = b % w;
+  return b - q + (q % 8u) * (unsigned)run + q / 8u;
 }
+constexpr int QUAD_RUN = 24;  // places per XCD visit in grids larger than the caches
 
 // Row and first node of block bx's thread; false past the end.
 __device__ __forceinline__ bool quad_at(const QuadGeom &g, int bx, int &j, int &k0) {
@@ -780,10 +777,8 @@ __device__ __forceinline__ void quad_cpml(const QuadCpml &cp, const QuadGeom &g,
 }
 
 template <bool OE, bool CP>
-__global__ void __launch_bounds__(256, QW)
-    h_update_quad(Fields f, Lanes L, QuadGeom g, QuadCpml cp) {
-  int i, bx;
-  if (!quad_block(g, i, bx)) return;
+__device__ __forceinline__ void h_quad(const Fields &f, const Lanes &L, const QuadGeom &g,
+                                       const QuadCpml &cp, int i, int bx) {
   int j, k0;
   const bool in = quad_at(g, bx, j, k0);
   bool fx = false, fy = false, fz = false;
@@ -836,10 +831,8 @@ __global__ void __launch_bounds__(256, QW)
 }
 
 template <bool OE, bool CP>
-__global__ void __launch_bounds__(256, QW)
-    e_update_quad(Fields f, Lanes L, QuadGeom g, QuadCpml cp) {
-  int i, bx;
-  if (!quad_block(g, i, bx)) return;
+__device__ __forceinline__ void e_quad(const Fields &f, const Lanes &L, const QuadGeom &g,
+                                       const QuadCpml &cp, int i, int bx) {
   int j, k0;
   const bool in = quad_at(g, bx, j, k0);
   bool fx = false, fy = false, fz = false;
@@ -891,6 +884,49 @@ __global__ void __launch_bounds__(256, QW)
   const int ne = min(4, nz - k0);
 #pragma unroll
   for (int a = 0; a < 3; a++) st_quad(f.u[a] + ip, vo, u[a], ne);
+}
+
+template <bool OE, bool CP>
+__global__ void __launch_bounds__(256, QW)
+    h_update_quad(Fields f, Lanes L, QuadGeom g, QuadCpml cp) {
+  const unsigned b = quad_order(blockIdx.x, g.run);
+  const int i = (int)(b / (unsigned)g.gx);
+  if (i < g.nx) h_quad<OE, CP>(f, L, g, cp, i, (int)(b - (unsigned)i * (unsigned)g.gx));
+}
+
+template <bool OE, bool CP>
+__global__ void __launch_bounds__(256, QW)
+    e_update_quad(Fields f, Lanes L, QuadGeom g, QuadCpml cp) {
+  const unsigned b = quad_order(blockIdx.x, g.run);
+  const int i = (int)(b / (unsigned)g.gx);
+  if (i < g.nx) e_quad<OE, CP>(f, L, g, cp, i, (int)(b - (unsigned)i * (unsigned)g.gx));
+}
+
+// The same over the models of a batch: what the kernels above take by
+// value, per model, and for each block its model.
+struct QuadModel {
+  Fields f;
+  Lanes L;
+  QuadGeom g[2];  // H, E
+  QuadCpml cp[2];
+  uint32_t first[2];  // the model's first block
+};
+
+template <bool OE, bool ESIDE>
+__global__ void __launch_bounds__(256, QW)
+    quad_batch(const QuadModel *__restrict__ ms, const uint32_t *__restrict__ model,
+               unsigned nblocks) {
+  const unsigned b = quad_order(blockIdx.x, QUAD_RUN);
+  if (b >= nblocks) return;
+  const QuadModel *m = ms + cload(model, b);
+  const QuadGeom g = cload(&m->g[ESIDE]);
+  const unsigned q = b - cload(&m->first[ESIDE]);
+  const int i = (int)(q / (unsigned)g.gx), bx = (int)(q - (unsigned)i * (unsigned)g.gx);
+  const Fields f = cload(&m->f);
+  const Lanes L = cload(&m->L);
+  const QuadCpml cp = cload(&m->cp[ESIDE]);
+  if (ESIDE) e_quad<OE, true>(f, L, g, cp, i, bx);
+  else h_quad<OE, true>(f, L, g, cp, i, bx);
 }
 
 // Loads/stores at a wave-uniform base plus a 32-bit per-lane byte offset,
@@ -2141,10 +2177,12 @@ __global__ void __launch_bounds__(256) gap_mid(Fields f, const DevOp *ops, int n
 // The post-E gap on the step result `f`. Fused steps keep the state before
 // the step in `fp` (the other buffer), whose u is u^n as pre_e reads it;
 // capture = 0 when the mid gap has already captured it. Segments as in
-// the mid gap; the last one advances the step counter.
+// the mid gap; the last one advances the step counter. Batches of unfused
+// steps have no mid gap: capture_next captures u^(n+1) for the next step
+// once the hooks have run.
 __device__ __forceinline__ void gap_post_e_body(Fields f, Fields fp, int capture, const DevOp *ops,
                                                 int nops, int q0, int q1, int last,
-                                                uint64_t *step) {
+                                                uint64_t *step, int capture_next = 0) {
   const uint64_t n = *step;
   const Gaps g = gaps_at(ops, nops, n);
   if (capture) {
@@ -2161,6 +2199,7 @@ __device__ __forceinline__ void gap_post_e_body(Fields f, Fields fp, int capture
     run_gap(f, ops, q0, q1, n, 1);
   }
   __syncthreads();
+  if (capture_next) lumped_capture(f, ops, nops);
   if (last && threadIdx.x == 0) *step = n + 1;
 }
 
@@ -2180,6 +2219,17 @@ struct GapArgs {
 __global__ void __launch_bounds__(256) gap_post_e_batch(const GapArgs *__restrict__ gs) {
   const GapArgs g = cload(gs, blockIdx.x);
   gap_post_e_body(g.f, g.fp, 1, g.ops, g.nops, 0, g.nops, 1, g.step);
+}
+
+// The same after unfused steps (u^n captured by the step before, and before
+// a run's first step by gap_capture_batch).
+__global__ void __launch_bounds__(256) gap_post_e_batch_quad(const GapArgs *__restrict__ gs) {
+  const GapArgs g = cload(gs, blockIdx.x);
+  gap_post_e_body(g.f, g.f, 0, g.ops, g.nops, 0, g.nops, 1, g.step, 1);
+}
+__global__ void __launch_bounds__(256) gap_capture_batch(const GapArgs *__restrict__ gs) {
+  const GapArgs g = cload(gs, blockIdx.x);
+  lumped_capture(g.f, g.ops, g.nops);
 }
 
 // ---- plane wave, total-field / scattered-field (planewave.rs) ----
@@ -3619,9 +3669,9 @@ QuadGeom quad_geom(const ems_gpu *h, int side, bool cpf, unsigned *blocks) {
   // 2.60 ms per step, 2.65 in plain order, 2.86 in contiguous eighths).
   const unsigned n = (unsigned)g.gx * (unsigned)g.nx;
   const bool cached = h->N * 24 <= ((size_t)256 << 20);
-  g.run = cached ? (int)((n + 7) / 8) : 24;
+  g.run = cached ? (int)((n + 7) / 8) : QUAD_RUN;
   const unsigned w = 8u * (unsigned)g.run;
-  *blocks = (n + w - 1) / w * w;
+  if (blocks) *blocks = (n + w - 1) / w * w;
   return g;
 }
 
@@ -6525,6 +6575,13 @@ struct ems_gpu_batch {
   uint32_t *d_seg = nullptr;
   size_t cap = 0;                 // models the device arrays hold
   int nblocks = 0;
+  // unfused quad steps (batch_quads): the models' arguments, each block's
+  // model (H, then E) and the numbers of blocks
+  bool quads = false;
+  QuadModel *d_qm = nullptr;
+  uint32_t *d_qmap = nullptr;
+  size_t qmap_cap = 0;
+  unsigned nqb[2] = {0, 0};
   hipGraphExec_t g1[2] = {nullptr, nullptr}, gK[2] = {nullptr, nullptr};
   int K = 16;                     // even
   bool graphs = true;             // ems_gpu_batch_set_graphs
@@ -6554,7 +6611,75 @@ void batch_drop_graphs(ems_gpu_batch *b) {
 }
 
 // Writes the per-model launch arguments of `act` for both parities.
+// Whether the batch steps with the quad kernels instead of the packed rows
+// (256 patch antennas, 30 M nodes of which the CPML holds 63 %: 1.13
+// against 1.24 ms a step; 8 antennas 50 against 74 us): every model's slabs
+// have to be the kernels' own to correct.
+bool batch_quads(const ems_gpu_batch *b, const std::vector<int> &act) {
+  if (!b->packed) return false;
+  for (int q : act) {
+    const ems_gpu *h = b->m[q];
+    QuadCpml cp;
+    if (!quad_ok(h) || !quad_cpml_args(h, 0, h->par, &cp) || !quad_cpml_args(h, 1, h->par, &cp))
+      return false;
+  }
+  return true;
+}
+
+int batch_quad_args(ems_gpu_batch *b, const std::vector<int> &act) {
+  const size_t n = act.size();
+  std::vector<QuadModel> qm(n);
+  std::vector<GapArgs> ga(n);
+  std::vector<uint32_t> map[2];
+  for (size_t q = 0; q < n; q++) {
+    ems_gpu *h = b->m[act[q]];
+    QuadModel &m = qm[q];
+    m.f = h->fb[h->par];
+    m.L = lanes_arg(h);
+    for (int side = 0; side < 2; side++) {
+      quad_cpml_args(h, side, h->par, &m.cp[side]);
+      m.g[side] = quad_geom(h, side, true, nullptr);
+      m.first[side] = (uint32_t)map[side].size();
+      map[side].resize(map[side].size() + (size_t)m.g[side].gx * m.g[side].nx, (uint32_t)q);
+    }
+    GapArgs &gg = ga[q];
+    gg.f = gg.fp = h->fb[h->par], gg.ops = h->d_ops, gg.nops = (int)h->ops.size();
+    gg.step = h->d_step;
+  }
+  if (n > b->cap) {
+    for (int p = 0; p < 2; p++) {
+      if (b->d_args[p]) BCK(b, hipFree(b->d_args[p]));
+      if (b->d_gap[p]) BCK(b, hipFree(b->d_gap[p]));
+      BCK(b, hipMalloc(&b->d_args[p], n * sizeof(FusedArgs)));
+      BCK(b, hipMalloc(&b->d_gap[p], n * sizeof(GapArgs)));
+    }
+    if (b->d_seg) BCK(b, hipFree(b->d_seg));
+    BCK(b, hipMalloc(&b->d_seg, (n + 1) * sizeof(uint32_t)));
+    if (b->d_qm) BCK(b, hipFree(b->d_qm));
+    b->d_qm = nullptr;
+    b->cap = n;
+  }
+  if (!b->d_qm) BCK(b, hipMalloc(&b->d_qm, b->cap * sizeof(QuadModel)));
+  const size_t nm = map[0].size() + map[1].size();
+  if (nm > b->qmap_cap) {
+    batch_drop_graphs(b);  // (they hold the table's address)
+    if (b->d_qmap) BCK(b, hipFree(b->d_qmap));
+    BCK(b, hipMalloc(&b->d_qmap, nm * sizeof(uint32_t)));
+    b->qmap_cap = nm;
+  }
+  for (int side = 0; side < 2; side++) {
+    if (b->nqb[side] != map[side].size()) batch_drop_graphs(b);  // (their launches' sizes)
+    b->nqb[side] = (unsigned)map[side].size();
+    BCK(b, hipMemcpy(b->d_qmap + (side ? map[0].size() : 0), map[side].data(),
+                     map[side].size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+  }
+  BCK(b, hipMemcpy(b->d_qm, qm.data(), n * sizeof(QuadModel), hipMemcpyHostToDevice));
+  BCK(b, hipMemcpy(b->d_gap[0], ga.data(), n * sizeof(GapArgs), hipMemcpyHostToDevice));
+  return 0;
+}
+
 int batch_args(ems_gpu_batch *b, const std::vector<int> &act) {
+  if (b->quads) return batch_quad_args(b, act);
   const size_t n = act.size();
   if (n > b->cap) {
     for (int p = 0; p < 2; p++) {
@@ -6565,6 +6690,8 @@ int batch_args(ems_gpu_batch *b, const std::vector<int> &act) {
     }
     if (b->d_seg) BCK(b, hipFree(b->d_seg));
     BCK(b, hipMalloc(&b->d_seg, (n + 1) * sizeof(uint32_t)));
+    if (b->d_qm) BCK(b, hipFree(b->d_qm));
+    b->d_qm = nullptr;
     b->cap = n;
   }
   std::vector<uint32_t> seg(n + 1, 0);
@@ -6610,7 +6737,50 @@ void batch_launch_tj(ems_gpu_batch *b, int par, int nm) {
 
 // One batched step from parity `par` (every active model holds its state
 // in fbuf[par]).
+// The models' dispersive media on the batch's stream (launch_poles).
+int batch_poles(ems_gpu_batch *b, const std::vector<int> &act, int stage, int par) {
+  for (int q : act) {
+    ems_gpu *h = b->m[q];
+    const hipStream_t own = h->stream;
+    h->stream = b->stream;
+    const int hp = par ^ h->boff;
+    const Fields &f = b->quads ? h->fb[h->par] : h->fb[hp ^ 1];
+    const int rc = launch_poles(h, stage, f, b->quads ? f : h->fb[hp], !b->quads);
+    h->stream = own;
+    if (rc) return bfail(b, rc, h->err);
+  }
+  return 0;
+}
+
+int batch_enqueue_quads(ems_gpu_batch *b, const std::vector<int> &act) {
+  const unsigned w = 8u * QUAD_RUN;
+  int rc;
+  const uint32_t *mh = b->d_qmap, *me = b->d_qmap + b->nqb[0];
+  const dim3 gh((b->nqb[0] + w - 1) / w * w), ge((b->nqb[1] + w - 1) / w * w);
+  if (b->oe)
+    hipLaunchKernelGGL((quad_batch<true, false>), gh, dim3(256), 0, b->stream,
+                       (const QuadModel *)b->d_qm, mh, b->nqb[0]);
+  else
+    hipLaunchKernelGGL((quad_batch<false, false>), gh, dim3(256), 0, b->stream,
+                       (const QuadModel *)b->d_qm, mh, b->nqb[0]);
+  BCK(b, hipGetLastError());
+  if ((rc = batch_poles(b, act, 0, 0))) return rc;
+  if (b->oe)
+    hipLaunchKernelGGL((quad_batch<true, true>), ge, dim3(256), 0, b->stream,
+                       (const QuadModel *)b->d_qm, me, b->nqb[1]);
+  else
+    hipLaunchKernelGGL((quad_batch<false, true>), ge, dim3(256), 0, b->stream,
+                       (const QuadModel *)b->d_qm, me, b->nqb[1]);
+  BCK(b, hipGetLastError());
+  if ((rc = batch_poles(b, act, 1, 0))) return rc;
+  hipLaunchKernelGGL(gap_post_e_batch_quad, dim3((unsigned)act.size()), dim3(256), 0, b->stream,
+                     (const GapArgs *)b->d_gap[0]);
+  BCK(b, hipGetLastError());
+  return 0;
+}
+
 int batch_enqueue_step(ems_gpu_batch *b, const std::vector<int> &act, int par) {
+  if (b->quads) return batch_enqueue_quads(b, act);
   const int nm = (int)act.size();
   const int key = b->packed ? (b->prefetch ? 1 : 0) : b->tj * 2 + (b->prefetch ? 1 : 0);
 #define BL(OE)                                                               \
@@ -6632,16 +6802,8 @@ int batch_enqueue_step(ems_gpu_batch *b, const std::vector<int> &act, int par) {
   }
 #undef BL
   BCK(b, hipGetLastError());
-  // Dispersive media of each model, on the batch stream.
-  for (int q : act) {
-    ems_gpu *h = b->m[q];
-    const hipStream_t own = h->stream;
-    h->stream = b->stream;
-    const int hp = par ^ h->boff;
-    const int rc = launch_poles(h, 1, h->fb[hp ^ 1], h->fb[hp], true);
-    h->stream = own;
-    if (rc) return bfail(b, rc, h->err);
-  }
+  int rc;
+  if ((rc = batch_poles(b, act, 1, par))) return rc;
   hipLaunchKernelGGL(gap_post_e_batch, dim3(nm), dim3(256), 0, b->stream,
                      (const GapArgs *)b->d_gap[par]);
   BCK(b, hipGetLastError());
@@ -6703,6 +6865,8 @@ void ems_gpu_batch_destroy(ems_gpu_batch *b) {
     if (b->d_args[p]) (void)hipFree(b->d_args[p]);
     if (b->d_gap[p]) (void)hipFree(b->d_gap[p]);
   }
+  if (b->d_qm) (void)hipFree(b->d_qm);
+  if (b->d_qmap) (void)hipFree(b->d_qmap);
   if (b->d_seg) (void)hipFree(b->d_seg);
   if (b->stream) (void)hipStreamDestroy(b->stream);
   delete b;
@@ -6770,10 +6934,20 @@ int ems_gpu_batch_run(ems_gpu_batch *b, const uint8_t *active, uint64_t n) {
                    "model " + std::to_string(q) + " has a coefficient pool of 4 GiB or more");
     BCK(b, hipStreamSynchronize(h->stream));
   }
-  if (boffs != b->boffs) batch_drop_graphs(b);  // (they hold the models' buffers)
+  const bool quads = batch_quads(b, act);
+  if (quads)  // in place: the models' buffers do not change over the run
+    for (size_t q = 0; q < act.size(); q++) boffs[q] = 2 + b->m[act[q]]->par;
+  // (graphs hold the models' buffers)
+  if (boffs != b->boffs || quads != b->quads) batch_drop_graphs(b);
   b->boffs = boffs;
+  b->quads = quads;
   int rc = batch_args(b, act);
   if (rc) return rc;
+  if (quads) {
+    hipLaunchKernelGGL(gap_capture_batch, dim3((unsigned)act.size()), dim3(256), 0, b->stream,
+                       (const GapArgs *)b->d_gap[0]);
+    BCK(b, hipGetLastError());
+  }
   if (!b->graphs) {  // the same launches, queued one by one
     int p = par;
     for (uint64_t s = 0; s < n; s++, p ^= 1)
@@ -6781,7 +6955,7 @@ int ems_gpu_batch_run(ems_gpu_batch *b, const uint8_t *active, uint64_t n) {
     BCK(b, hipStreamSynchronize(b->stream));
     for (int q : act) {
       ems_gpu *h = b->m[q];
-      h->par = p ^ h->boff;
+      if (!quads) h->par = p ^ h->boff;
       advance_counts(h, n);
     }
     return EMS_OK;
@@ -6808,7 +6982,7 @@ int ems_gpu_batch_run(ems_gpu_batch *b, const uint8_t *active, uint64_t n) {
   BCK(b, hipStreamSynchronize(b->stream));
   for (int q : act) {
     ems_gpu *h = b->m[q];
-    h->par = p ^ h->boff;
+    if (!quads) h->par = p ^ h->boff;
     advance_counts(h, n);
   }
   return EMS_OK;

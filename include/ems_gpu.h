@@ -391,8 +391,10 @@ int ems_gpu_batch_create(ems_gpu *const *models, int n, ems_gpu_batch **out);
 void ems_gpu_batch_destroy(ems_gpu_batch *b);
 const char *ems_gpu_batch_last_error(const ems_gpu_batch *b);
 /* Kernel for every model of the batch: mode 1 the tiled fused kernel, 2
- * the same without the next-plane prefetch, 4 packed short rows (every
- * model nz <= 64), 5 packed without the prefetch; tile height (3, 7, 15;
+ * the same without the next-plane prefetch, 4 and 5 short rows (every model
+ * nz <= 64): the unfused kernels of four nodes per thread, or, where a
+ * model's CPML slabs are not in their form (ems_gpu_set_unfused_prefetch),
+ * packed fused rows (5 without the prefetch); tile height (3, 7, 15;
  * tiled modes only), x chunks per model (0 automatic). */
 int ems_gpu_batch_set_schedule(ems_gpu_batch *b, int mode, int tile_rows, int x_chunks);
 /* n steps of the models with active[q] != 0 (NULL: all); returns after
