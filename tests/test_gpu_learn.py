@@ -154,3 +154,55 @@ def test_invalid_arguments():
     with pytest.raises(EmsError):
         n.train_batch([0, 4], 0, 1e-3)
     n.close()
+
+
+# Shapes at the edges of the convolutions' tiles: single samples and
+# channels, channels past and short of 16, 32 and 64, dilations that do not
+# divide the length, that exceed a block and that exceed the sequence, and
+# lengths around a block's 64 samples.
+EDGES = [(1, 1, 1, (1, 1), 1, 1), (5, 3, 33, (3, 40), 2, 257), (4, 2, 48, (1, 2, 64, 100), 3, 130),
+         (17, 18, 70, (7, 65, 200), 2, 96), (4, 2, 130, (2, 31), 1, 65), (2, 1, 32, (5, 1), 9, 63),
+         (4, 2, 64, (1, 2, 4, 8, 16, 32), 5, 500)]
+
+
+@pytest.mark.parametrize("shape", EDGES)
+def test_edge_shapes_match_oracle(shape):
+    """Outputs and gradients against the oracle, the tolerances of the tests
+    above (sums of up to 9 * 130 products in f32, in another order)."""
+    cin, cout, ch, dil, B, T = shape
+    n = _net(cin, cout, ch, dil, 11)
+    s = O.Shape(cin, cout, ch, dil)
+    rng = np.random.default_rng(T)
+    p = n.params() + rng.standard_normal(s.count).astype(np.float32) * 0.02
+    n.set_params(p)
+    x = rng.standard_normal((B, cin, T)).astype(np.float32)
+    y = rng.standard_normal((B, cout, T)).astype(np.float32)
+    _close(n.forward(x), O.forward(s, p.astype(np.float64), x.astype(np.float64)), 2e-5)
+    for b in (B, 1):  # (the second call in buffers sized for the first)
+        loss, g = n.loss_grad(x[:b], y[:b], T // 3)
+        lo, go = O.loss_and_grad(s, p.astype(np.float64), x[:b].astype(np.float64),
+                                 y[:b].astype(np.float64), T // 3)
+        assert abs(loss - lo) <= 1e-5 * abs(lo)
+        for l in range(s.L):
+            _close(g[s.woff[l]:s.boff[l]], go[s.woff[l]:s.boff[l]], 2e-4)
+            _close(g[s.boff[l]:s.boff[l] + s.lo[l]], go[s.boff[l]:s.boff[l] + s.lo[l]], 2e-4)
+    # more sequences than the first calls, shorter ones
+    z = rng.standard_normal((4 * B + 1, cin, max(1, T // 4))).astype(np.float32)
+    _close(n.forward(z), O.forward(s, p.astype(np.float64), z.astype(np.float64)), 2e-5)
+    n.close()
+
+
+def test_infinite_and_tiny_inputs():
+    """An infinite sample saturates tanh as the plain sums do; samples at the
+    bottom of f32's range do not disturb the others."""
+    dil = (1, 2)
+    n = _net(2, 1, 40, dil, 3)
+    s = O.Shape(2, 1, 40, dil)
+    p = n.params()
+    x = np.random.default_rng(2).standard_normal((2, 2, 90)).astype(np.float32)
+    x[0, 0, 17] = np.inf
+    x[1, 1, 40:50] = np.float32(1e-42)
+    got = n.forward(x)
+    assert np.all(np.isfinite(got))
+    _close(got, O.forward(s, p.astype(np.float64), x.astype(np.float64)), 2e-5)
+    n.close()
