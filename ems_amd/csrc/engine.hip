@@ -539,7 +539,7 @@ __device__ __forceinline__ void cpml_node(const FSlab *__restrict__ slabs, uint3
 // registration order with the very expressions of cpml_slab, instead of in
 // launches of their own (513^3 nodes: 0.1 ms per half-step for 9 % of the
 // nodes; the psi loads are issued with the fields').
-constexpr int QW = 5;  // waves per SIMD the quad kernels are held to (90 VGPRs with CPML)
+constexpr int QW = 4;  // waves per SIMD the quad kernels are held to (127 VGPRs with CPML)
 constexpr size_t QUAD_PAD = 4;  // floats of padding behind (psi: around) quad-read arrays
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
@@ -615,12 +615,14 @@ __device__ __forceinline__ bool quad_at(const QuadGeom &g, int bx, int &j, int &
 // corrections of a component come in the order of its normals; other slabs
 // are corrected by launches of their own). An absent end has hi <= lo.
 struct CpmlEnd {
-  float *psi;        // box (i, j, k) order
-  const float *bak;  // b, a, k by depth, each (hi - lo) + 2 QUAD_PAD apart
-  int lo, hi;        // along the normal
+  float *psi;  // box (i, j, k) order
+  int lo, hi;  // along the normal
 };
 struct QuadCpml {
-  CpmlEnd e[3][2][2];  // component, which of its normals, low / high end
+  CpmlEnd e[3][2][2];       // component, which of its normals, low / high end
+  // per normal and end: b, a, k by depth, each (hi - lo) + 2 QUAD_PAD apart
+  // (the two components' are equal: quad_cpml_args)
+  const float *bak[3][2];
 };
 constexpr int pair_of(int c, int n) { return c == 0 ? n - 1 : (c == 1 ? n / 2 : n); }
 
@@ -630,7 +632,6 @@ struct QuadPair {
   bool in;
   int lo, hi;
   GAS float *psi;
-  const float *bak;
 };
 template <bool ESIDE, int C, int N>
 __device__ __forceinline__ QuadPair quad_pair(const QuadCpml &cp, const QuadGeom &g, int i, int j,
@@ -644,7 +645,6 @@ __device__ __forceinline__ QuadPair quad_pair(const QuadCpml &cp, const QuadGeom
   q.lo = hi ? B.lo : A.lo, q.hi = hi ? B.hi : A.hi;
   q.in = N == 2 ? (pos + 4 > q.lo && pos < q.hi) : (pos >= q.lo && pos < q.hi);
   q.in = q.in && (N == 0 || i < ex) && (N == 1 || j < ey) && (N == 2 || k0 < ez);
-  q.bak = hi ? B.bak : A.bak;
   GAS float *psi = (GAS float *)(hi ? B.psi : A.psi);
   if (N == 0) psi += (ptrdiff_t)((size_t)(i - q.lo) * ey) * ez + (j * ez + k0);
   if (N == 1) psi += (ptrdiff_t)((size_t)i * (q.hi - q.lo) + (j - q.lo)) * ez + k0;
@@ -653,48 +653,84 @@ __device__ __forceinline__ QuadPair quad_pair(const QuadCpml &cp, const QuadGeom
   return q;
 }
 
+// What the corrections of a quad read, loaded with the plane's fields so
+// that all the latencies overlap: psi per (component, normal), b, a, k per
+// normal (wave-uniform for x). Costs a wave per SIMD (90 to 127 VGPRs) and
+// is worth it from the smallest to the largest: 131 x 97 x 74 with 8-node
+// slabs 41.0 to 37.2 us a step, 513^3 2.605 to 2.591 ms, 256 patch antennas
+// 1132 to 1088 us.
+struct QuadPre {
+  f4 psi[3][2];
+  float xb, xa, xk, yb, ya, yk;
+  f4 zb, za, zk;
+};
 template <bool ESIDE, int C, int N>
-__device__ __forceinline__ f4 quad_psi(const QuadCpml &cp, const QuadGeom &g, int i, int j,
-                                       int k0) {
+__device__ __forceinline__ void quad_psi(const QuadCpml &cp, const QuadGeom &g, int i, int j,
+                                         int k0, QuadPre &P) {
   const QuadPair q = quad_pair<ESIDE, C, N>(cp, g, i, j, k0);
-  f4 p = {0.0f, 0.0f, 0.0f, 0.0f};
-  if (q.in) p = *(const GAS f4u *)q.psi;
-  return p;
+  if (q.in) P.psi[C][pair_of(C, N)] = *(const GAS f4u *)q.psi;
+}
+// (The tables of one normal take the box of either component: they agree
+// along it.)
+template <bool ESIDE>
+__device__ __forceinline__ void quad_pre(const QuadCpml &cp, const QuadGeom &g, bool fx, bool fy,
+                                         bool fz, int i, int j, int k0, QuadPre &P) {
+  if (fx) {
+    const bool hi = i >= cp.e[1][0][1].lo;
+    const int lo = hi ? cp.e[1][0][1].lo : cp.e[1][0][0].lo;
+    const int D = (hi ? cp.e[1][0][1].hi : cp.e[1][0][0].hi) - lo + 2 * (int)QUAD_PAD;
+    const float *b = (hi ? cp.bak[0][1] : cp.bak[0][0]) + (i - lo);
+    P.xb = cload(b), P.xa = cload(b, D), P.xk = cload(b, 2 * D);
+    quad_psi<ESIDE, 1, 0>(cp, g, i, j, k0, P);
+    quad_psi<ESIDE, 2, 0>(cp, g, i, j, k0, P);
+  }
+  if (fy) {
+    const QuadPair q = quad_pair<ESIDE, 2, 1>(cp, g, 0, j, 0);
+    if (q.in) {
+      const bool hi = j >= cp.e[2][1][1].lo;
+      const int D = q.hi - q.lo + 2 * (int)QUAD_PAD;
+      const GAS float *b = (const GAS float *)(hi ? cp.bak[1][1] : cp.bak[1][0]) + (j - q.lo);
+      P.yb = b[0], P.ya = b[D], P.yk = b[2 * D];
+    }
+    quad_psi<ESIDE, 0, 1>(cp, g, i, j, k0, P);
+    quad_psi<ESIDE, 2, 1>(cp, g, i, j, k0, P);
+  }
+  if (fz) {
+    const QuadPair q = quad_pair<ESIDE, 1, 2>(cp, g, 0, 0, k0);
+    if (q.in) {
+      const bool hi = k0 + 4 > cp.e[1][1][1].lo;
+      const int D = q.hi - q.lo + 2 * (int)QUAD_PAD;
+      const GAS float *b = (const GAS float *)(hi ? cp.bak[2][1] : cp.bak[2][0]) + (k0 - q.lo);
+      P.zb = *(const GAS f4u *)b, P.za = *(const GAS f4u *)(b + D);
+      P.zk = *(const GAS f4u *)(b + 2 * D);
+    }
+    quad_psi<ESIDE, 0, 2>(cp, g, i, j, k0, P);
+    quad_psi<ESIDE, 1, 2>(cp, g, i, j, k0, P);
+  }
 }
 
 // The pair's correction of a quad (cpml.rs:495-543): component t with
-// coefficient cf, d the derivative's difference h - l, pin its psi.
-// Elements outside the slab keep their value and psi.
+// coefficient cf, d the derivative's difference h - l. Elements outside the
+// slab keep their value and psi.
 template <bool ESIDE, int C, int N>
 __device__ __forceinline__ void quad_cpml_apply(const QuadCpml &cp, const QuadGeom &g, int i,
-                                                int j, int k0, f4 pin, f4 d, f4 cf, f4 &t) {
+                                                int j, int k0, const QuadPre &P, f4 d, f4 cf,
+                                                f4 &t) {
   const QuadPair q = quad_pair<ESIDE, C, N>(cp, g, i, j, k0);
   if (!q.in) return;
-  const int D = q.hi - q.lo + 2 * (int)QUAD_PAD;
-  f4 bz, az, kz;
-  if (N == 2) {
-    const GAS float *b = (const GAS float *)q.bak + (k0 - q.lo);
-    bz = *(const GAS f4u *)b, az = *(const GAS f4u *)(b + D), kz = *(const GAS f4u *)(b + 2 * D);
-  } else {
-    float b1, a1, k1;
-    if (N == 0) {
-      const float *b = q.bak + (i - q.lo);
-      b1 = cload(b), a1 = cload(b, D), k1 = cload(b, 2 * D);
-    } else {
-      const GAS float *b = (const GAS float *)q.bak + (j - q.lo);
-      b1 = b[0], a1 = b[D], k1 = b[2 * D];
-    }
-    bz = f4{b1, b1, b1, b1}, az = f4{a1, a1, a1, a1}, kz = f4{k1, k1, k1, k1};
-  }
   const float sign = N == (C + 1) % 3 ? 1.0f : -1.0f, scale = ESIDE ? 1.0f : -1.0f;
   const int ez = g.nz - ((ESIDE == (C == 2)) ? 1 : 0);
   const int k_lo = N == 2 ? q.lo : 0, k_hi = N == 2 ? q.hi : ez;
+  const f4 pin = P.psi[C][pair_of(C, N)];
   f4 ps;
 #pragma unroll
   for (int e = 0; e < 4; e++) {
+    const float b = N == 0 ? P.xb : (N == 1 ? P.yb : P.zb[e]);
+    const float a = N == 0 ? P.xa : (N == 1 ? P.ya : P.za[e]);
+    const float kk = N == 0 ? P.xk : (N == 1 ? P.yk : P.zk[e]);
     const float sv = sign * d[e];
-    ps[e] = flush(bz[e] * pin[e] + az[e] * sv);
-    const float tn = flush(t[e] + scale * cf[e] * (kz[e] * sv + ps[e]));
+    ps[e] = flush(b * pin[e] + a * sv);
+    const float tn = flush(t[e] + scale * cf[e] * (kk * sv + ps[e]));
     t[e] = (k0 + e >= k_lo && k0 + e < k_hi) ? tn : t[e];
   }
   if (k0 >= k_lo && k0 + 4 <= k_hi) {
@@ -725,54 +761,25 @@ __device__ __forceinline__ bool quad_x_slab(const QuadCpml &cp, int i) {
   return in;
 }
 
-// The psi of the first normal whose slabs the wave meets (two components),
-// loaded with the plane's fields so that the latencies overlap; the other
-// normals' (at the grid's edges and corners) are loaded when their turn
-// comes.
-template <bool ESIDE>
-__device__ __forceinline__ void quad_psi_first(const QuadCpml &cp, const QuadGeom &g, bool fx,
-                                               bool fy, int i, int j, int k0, f4 P[2]) {
-  if (fx) {
-    P[0] = quad_psi<ESIDE, 1, 0>(cp, g, i, j, k0);
-    P[1] = quad_psi<ESIDE, 2, 0>(cp, g, i, j, k0);
-  } else if (fy) {
-    P[0] = quad_psi<ESIDE, 0, 1>(cp, g, i, j, k0);
-    P[1] = quad_psi<ESIDE, 2, 1>(cp, g, i, j, k0);
-  } else {
-    P[0] = quad_psi<ESIDE, 0, 2>(cp, g, i, j, k0);
-    P[1] = quad_psi<ESIDE, 1, 2>(cp, g, i, j, k0);
-  }
-}
-
 // Every correction of a quad; d<c><n> the difference along normal n that
 // component c uses.
 template <bool ESIDE>
 __device__ __forceinline__ void quad_cpml(const QuadCpml &cp, const QuadGeom &g, bool fx, bool fy,
-                                          bool fz, int i, int j, int k0, const f4 P[2],
+                                          bool fz, int i, int j, int k0, const QuadPre &P,
                                           const f4 &d01, const f4 &d02, const f4 &d10,
                                           const f4 &d12, const f4 &d20, const f4 &d21,
                                           const f4 cf[3], f4 t[3]) {
   if (fx) {
-    quad_cpml_apply<ESIDE, 1, 0>(cp, g, i, j, k0, P[0], d10, cf[1], t[1]);
-    quad_cpml_apply<ESIDE, 2, 0>(cp, g, i, j, k0, P[1], d20, cf[2], t[2]);
+    quad_cpml_apply<ESIDE, 1, 0>(cp, g, i, j, k0, P, d10, cf[1], t[1]);
+    quad_cpml_apply<ESIDE, 2, 0>(cp, g, i, j, k0, P, d20, cf[2], t[2]);
   }
   if (fy) {
-    f4 p0 = P[0], p1 = P[1];
-    if (fx) {
-      p0 = quad_psi<ESIDE, 0, 1>(cp, g, i, j, k0);
-      p1 = quad_psi<ESIDE, 2, 1>(cp, g, i, j, k0);
-    }
-    quad_cpml_apply<ESIDE, 0, 1>(cp, g, i, j, k0, p0, d01, cf[0], t[0]);
-    quad_cpml_apply<ESIDE, 2, 1>(cp, g, i, j, k0, p1, d21, cf[2], t[2]);
+    quad_cpml_apply<ESIDE, 0, 1>(cp, g, i, j, k0, P, d01, cf[0], t[0]);
+    quad_cpml_apply<ESIDE, 2, 1>(cp, g, i, j, k0, P, d21, cf[2], t[2]);
   }
   if (fz) {
-    f4 p0 = P[0], p1 = P[1];
-    if (fx || fy) {
-      p0 = quad_psi<ESIDE, 0, 2>(cp, g, i, j, k0);
-      p1 = quad_psi<ESIDE, 1, 2>(cp, g, i, j, k0);
-    }
-    quad_cpml_apply<ESIDE, 0, 2>(cp, g, i, j, k0, p0, d02, cf[0], t[0]);
-    quad_cpml_apply<ESIDE, 1, 2>(cp, g, i, j, k0, p1, d12, cf[1], t[1]);
+    quad_cpml_apply<ESIDE, 0, 2>(cp, g, i, j, k0, P, d02, cf[0], t[0]);
+    quad_cpml_apply<ESIDE, 1, 2>(cp, g, i, j, k0, P, d12, cf[1], t[1]);
   }
 }
 
@@ -794,8 +801,8 @@ __device__ __forceinline__ void h_quad(const Fields &f, const Lanes &L, const Qu
   const unsigned vo = 4u * (unsigned)(j * nz + k0);
   const unsigned vj = jv ? vo + 4u * (unsigned)nz : vo;
   const unsigned ve = k0 + 4 < nz ? vo + 16u : vo;  // the node after the quad
-  f4 P[2];
-  if (CP && (fx || fy || fz)) quad_psi_first<false>(cp, g, fx, fy, i, j, k0, P);
+  QuadPre P;
+  if (CP && (fx || fy || fz)) quad_pre<false>(cp, g, fx, fy, fz, i, j, k0, P);
   const f4 ux = ld4(f.u[0] + ip, vo), uy = ld4(f.u[1] + ip, vo), uz = ld4(f.u[2] + ip, vo);
   const float uxe = ld1(f.u[0] + ip, ve), uye = ld1(f.u[1] + ip, ve);
   const f4 uxj = ld4(f.u[0] + ip, vj), uzj = ld4(f.u[2] + ip, vj);
@@ -849,8 +856,8 @@ __device__ __forceinline__ void e_quad(const Fields &f, const Lanes &L, const Qu
   const unsigned vj = j > 0 ? vo - 4u * (unsigned)nz : vo;
   const unsigned ve = k0 > 0 ? vo - 4u : vo;  // the node before the quad
   const f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-  f4 P[2];
-  if (CP && (fx || fy || fz)) quad_psi_first<true>(cp, g, fx, fy, i, j, k0, P);
+  QuadPre P;
+  if (CP && (fx || fy || fz)) quad_pre<true>(cp, g, fx, fy, fz, i, j, k0, P);
   const f4 ix = ld4(f.i[0] + ip, vo), iy = ld4(f.i[1] + ip, vo), iz = ld4(f.i[2] + ip, vo);
   float ixe = ld1(f.i[0] + ip, ve), iye = ld1(f.i[1] + ip, ve);
   f4 ixj = ld4(f.i[0] + ip, vj), izj = ld4(f.i[2] + ip, vj);
@@ -3297,6 +3304,7 @@ __global__ void __launch_bounds__(64) energy_combine_many(const EnergyModel *__r
 struct HostSlab {
   SlabArg arg;  // arg.psi is set per launch (parity)
   float *d_b = nullptr, *d_a = nullptr, *d_k = nullptr;
+  std::vector<float> bak;  // their values, as d_b holds them
   float *d_psi[2] = {nullptr, nullptr};  // H side: double-buffered; E side: [0] only
   float *d_delta = nullptr;  // H side, run outside the fused kernel: its increments
   size_t len = 0;
@@ -3597,7 +3605,9 @@ bool quad_cpml_args(const ems_gpu *h, int side, int par, QuadCpml *out) {
   QuadCpml cp;
   for (auto &c : cp.e)
     for (auto &n : c)
-      for (auto &e : n) e = CpmlEnd{nullptr, nullptr, INT32_MAX / 2, 0};
+      for (auto &e : n) e = CpmlEnd{nullptr, INT32_MAX / 2, 0};
+  for (auto &n : cp.bak) n[0] = n[1] = nullptr;
+  const HostSlab *own[3][2][2] = {};  // by component and normal, as cp.e
   for (auto &s : h->slabs) {
     const SlabArg &a = s.arg;
     if (s.len == 0 || a.e_side != side) continue;
@@ -3613,19 +3623,32 @@ bool quad_cpml_args(const ems_gpu *h, int side, int par, QuadCpml *out) {
     if (w == 0)  // (the second normal's corrections follow the first's)
       for (auto &e : cp.e[a.comp][1])
         if (e.psi) return false;
-    CpmlEnd in{s.d_psi[side ? 0 : par], s.d_b, a.lo[a.normal], a.hi[a.normal]};
+    CpmlEnd in{s.d_psi[side ? 0 : par], a.lo[a.normal], a.hi[a.normal]};
+    const HostSlab **o = own[a.comp][w];
     if (!lo.psi) {
-      lo = in;
+      lo = in, o[0] = &s;
     } else if (!hi.psi) {
-      hi = in;
-      if (hi.lo < lo.lo) std::swap(lo, hi);
+      hi = in, o[1] = &s;
+      if (hi.lo < lo.lo) std::swap(lo, hi), std::swap(o[0], o[1]);
       const int gap = a.normal == 2 ? hi.lo / 4 * 4 : hi.lo;  // (whole quads along z)
       if (gap < lo.hi) return false;
     } else {
       return false;
     }
   }
-  // a lone slab is the low end; the absent high end starts past the grid
+  // (a lone slab is the low end; the absent high end starts past the grid)
+  // The two components of a normal: the same ends, boxes along it and
+  // tables.
+  for (int n = 0; n < 3; n++)
+    for (int e = 0; e < 2; e++) {
+      const int c1 = n == 0 ? 1 : 0, c2 = n == 2 ? 1 : 2;
+      const HostSlab *x = own[c1][pair_of(c1, n)][e], *y = own[c2][pair_of(c2, n)][e];
+      if (!x && !y) continue;
+      if (!x || !y || x->arg.lo[n] != y->arg.lo[n] || x->arg.hi[n] != y->arg.hi[n] ||
+          x->bak != y->bak)
+        return false;
+      cp.bak[n][e] = x->d_b;
+    }
   *out = cp;
   return true;
 }
@@ -4980,6 +5003,7 @@ int ems_gpu_add_cpml(ems_gpu *h, const ems_cpml_slab *s, int n) {
     }
     if ((rc = upload_padded(h, &hs.d_b, bak.data() + QUAD_PAD, 3 * seg - 2 * QUAD_PAD))) return rc;
     hs.d_a = hs.d_b + seg, hs.d_k = hs.d_a + seg;
+    hs.bak = std::move(bak);
     hs.len = (size_t)(in.hi[0] - in.lo[0]) * (in.hi[1] - in.lo[1]) * (in.hi[2] - in.lo[2]);
     for (int b = 0; b < (a.e_side ? 1 : 2); b++)
       if ((rc = upload_padded(h, &hs.d_psi[b], nullptr, hs.len))) return rc;
