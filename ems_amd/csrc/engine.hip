@@ -2393,99 +2393,146 @@ __host__ __device__ __forceinline__ size_t mf_lds_need(uint32_t nr, uint64_t nev
 }
 
 // LDS bytes of a narrow block's image (envelopes at most 3 below the
-// diagonal): per row 4 envelope values, 3 column values, x, a packed word.
+// diagonal): per row (up to a multiple of 4) three envelope values, the
+// diagonal and its reciprocal, x, and three column values.
 __host__ __device__ __forceinline__ size_t mf_narrow_need(uint32_t nr) {
-  return 68 * (size_t)nr;
+  return 72 * (size_t)((nr + 3) / 4 * 4);
 }
 
-// One narrow block by a wave: the lanes stage each row's envelope (len =
-// i - f + 1 <= 4 values), its column (up to 3 rows k = j + dk, decreasing)
-// and right-hand side; lane 0 then substitutes with the last three solved
-// values in registers and the next row's data loaded one row ahead, the
-// terms in the row form's order (ascending j forward, decreasing k
-// backward).
-__device__ __forceinline__ void mf_narrow(const DevMerged &m, uint32_t r0, uint32_t nr,
-                                          double *xs) {
-  double *rv = xs, *cw = rv + 4 * (size_t)nr, *x = cw + 3 * (size_t)nr;
-  uint32_t *meta = (uint32_t *)(x + nr);
-  for (uint32_t i = threadIdx.x; i < nr; i += 64) {
-    const uint32_t f = m.ef[r0 + i], len = i - f + 1;
-    const uint64_t e = m.eo[r0 + i];
-    for (uint32_t t = 0; t < len; t++) rv[4 * (size_t)i + t] = m.ev[e + t];
-    const uint32_t q0 = m.cs[r0 + i], nc = m.cs[r0 + i + 1] - q0;
-    uint32_t w = len | (nc << 4);
-    for (uint32_t t = 0; t < nc; t++) {
-      cw[3 * (size_t)i + t] = m.cv[q0 + t];
-      w |= (m.cr[q0 + t] - i) << (8 + 2 * t);
+// The wave's own writes (LDS and memory) before its reads after it. (Blocks
+// are solved by single waves, several of them in one thread block.)
+__device__ __forceinline__ void mf_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// s / d by d's correctly rounded reciprocal r: the product s r corrected by
+// its exact remainder twice; the first correction is within an ulp of the
+// quotient, the second is then correctly rounded (Markstein, "Computation of
+// elementary functions on the IBM RISC System/6000 processor", IBM J. Res.
+// Dev. 34, 1990), so this is the IEEE quotient wherever nothing over- or
+// underflows (mf_in_range), in half the dependent operations. A zero
+// quotient may have the other sign; the currents flush it to +0.
+__device__ __forceinline__ double mf_div(double s, double d, double r) {
+  const double q = s * r;
+  const double q1 = __builtin_fma(__builtin_fma(-q, d, s), r, q);
+  return __builtin_fma(__builtin_fma(-q1, d, s), r, q1);
+}
+__device__ __forceinline__ bool mf_in_range(double s) {
+  const double a = fabs(s);
+  return (a >= 0x1p-900 && a <= 0x1p900) || s == 0.0;
+}
+
+// One narrow block by a wave: the lanes stage each row's terms in fixed
+// places (zeros where the envelope or the column is shorter: s - 0 x is s),
+// the diagonal's reciprocal and the right-hand side; lane 0 then substitutes
+// with the last three solved values in registers, four rows' data loaded
+// ahead, the terms in the row form's order (ascending j forward, decreasing
+// k backward). Rows past the end solve 0 = 0. Returns false (x not written)
+// where a value leaves mf_div's range or is not finite.
+//
+// Bound by the chain of one row after the other: a product, a subtraction
+// and the quotient's five dependent operations per row and direction (some
+// 330 rows: 77 us; with an IEEE division, the row's length tested and one
+// row loaded ahead 97, and the large blocks' launch before it).
+__device__ __forceinline__ bool mf_narrow(const DevMerged &m, uint32_t r0, uint32_t nr,
+                                          double *xs, uint32_t lane) {
+  const uint32_t n4 = (nr + 3) / 4 * 4;
+  double *ra = xs;                      // [row][6]: a (of x[i-3], x[i-2], x[i-1]), 1/d, d, x
+  double *rc = ra + 6 * (size_t)n4;     // [row][3]: the column at j + 3, j + 2, j + 1
+  bool ok = true;
+  for (uint32_t i = lane; i < n4; i += 64) {
+    double a[3] = {0.0, 0.0, 0.0}, c[3] = {0.0, 0.0, 0.0}, d = 1.0, y = 0.0;
+    if (i < nr) {
+      const uint32_t f = m.ef[r0 + i], len = i - f;  // (<= 3 off the diagonal)
+      const uint64_t e = m.eo[r0 + i];
+      for (uint32_t t = 0; t < 3; t++)
+        if (t >= 3 - len) a[t] = m.ev[e + t - (3 - len)];
+      d = m.ev[e + len];
+      const uint32_t q1 = m.cs[r0 + i + 1];
+      for (uint32_t q = m.cs[r0 + i]; q < q1; q++) {
+        const uint32_t dk = m.cr[q] - i;
+        const double v = m.cv[q];
+        c[0] = dk == 3 ? v : c[0], c[1] = dk == 2 ? v : c[1], c[2] = dk == 1 ? v : c[2];
+      }
+      y = mf_rhs(m, r0, i, m.cur, m.circ);
     }
-    meta[i] = w;
-    x[i] = mf_rhs(m, r0, i, m.cur, m.circ);
+    const double ad = fabs(d);
+    ok = ok && ad >= 0x1p-100 && ad <= 0x1p100;
+    double *o = ra + 6 * (size_t)i;
+    o[0] = a[0], o[1] = a[1], o[2] = a[2], o[3] = 1.0 / d, o[4] = d, o[5] = y;
+    double *oc = rc + 3 * (size_t)i;
+    oc[0] = c[0], oc[1] = c[1], oc[2] = c[2];
   }
-  __syncthreads();
-  if (threadIdx.x == 0) {
+  mf_sync();
+  if (lane == 0 && n4) {
     double w1 = 0.0, w2 = 0.0, w3 = 0.0;
-    uint32_t mt = meta[0];
-    double a0 = rv[0], a1 = rv[1], a2 = rv[2], a3 = rv[3], y = x[0];
-    for (uint32_t i = 0; i < nr; i++) {
-      const uint32_t len = mt & 7;
-      const double b0 = a0, b1 = a1, b2 = a2, b3 = a3;
-      double s = y;
-      if (i + 1 < nr) {
-        const double *r = rv + 4 * (size_t)(i + 1);
-        mt = meta[i + 1], a0 = r[0], a1 = r[1], a2 = r[2], a3 = r[3], y = x[i + 1];
+    double v[4][6], t[4][6];
+    auto rows = [&](uint32_t i, double b[][6]) {
+#pragma unroll
+      for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int e = 0; e < 6; e++) b[u][e] = ra[6 * (size_t)(i + u) + e];
+    };
+    rows(0, v);
+    for (uint32_t i = 0; i < n4; i += 4) {
+      rows(i + 4 < n4 ? i + 4 : i, t);
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        double q = v[u][5];
+        q -= v[u][0] * w3;
+        q -= v[u][1] * w2;
+        q -= v[u][2] * w1;
+        ok = ok && mf_in_range(q);
+        const double x = mf_div(q, v[u][4], v[u][3]);
+        ra[6 * (size_t)(i + u) + 5] = x;
+        w3 = w2, w2 = w1, w1 = x;
       }
-      double d;
-      if (len == 4) {
-        s -= b0 * w3;
-        s -= b1 * w2;
-        s -= b2 * w1;
-        d = b3;
-      } else if (len == 3) {
-        s -= b0 * w2;
-        s -= b1 * w1;
-        d = b2;
-      } else if (len == 2) {
-        s -= b0 * w1;
-        d = b1;
-      } else {
-        d = b0;
-      }
-      const double xi = s / d;
-      x[i] = xi;
-      w3 = w2, w2 = w1, w1 = xi;
+#pragma unroll
+      for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int e = 0; e < 6; e++) v[u][e] = t[u][e];
     }
     // backward: w1, w2, w3 = x[j + 1], x[j + 2], x[j + 3]
     w1 = w2 = w3 = 0.0;
-    const uint32_t jl = nr - 1;
-    mt = meta[jl];
-    double c0 = cw[3 * (size_t)jl], c1 = cw[3 * (size_t)jl + 1], c2 = cw[3 * (size_t)jl + 2];
-    double dg = rv[4 * (size_t)jl + (mt & 7) - 1];
-    y = x[jl];
-    for (uint32_t j = nr; j-- > 0;) {
-      const uint32_t nc = (mt >> 4) & 3, dk = mt >> 8;
-      const double e0 = c0, e1 = c1, e2 = c2, dj = dg;
-      double s = y;
-      if (j > 0) {
-        const uint32_t jn = j - 1;
-        mt = meta[jn];
-        c0 = cw[3 * (size_t)jn], c1 = cw[3 * (size_t)jn + 1], c2 = cw[3 * (size_t)jn + 2];
-        dg = rv[4 * (size_t)jn + (mt & 7) - 1];
-        y = x[jn];
+    double c[4][3], ct[4][3];
+    auto cols = [&](uint32_t i, double b[][6], double g[][3]) {
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+#pragma unroll
+        for (int e = 3; e < 6; e++) b[u][e] = ra[6 * (size_t)(i + u) + e];
+#pragma unroll
+        for (int e = 0; e < 3; e++) g[u][e] = rc[3 * (size_t)(i + u) + e];
       }
-      const double ev[3] = {e0, e1, e2};
-      for (uint32_t t = 0; t < 3; t++) {
-        if (t >= nc) break;
-        const uint32_t k = (dk >> (2 * t)) & 3;
-        s -= ev[t] * (k == 1 ? w1 : (k == 2 ? w2 : w3));
+    };
+    cols(n4 - 4, v, c);
+    for (uint32_t j = n4; j > 0; j -= 4) {
+      cols(j > 4 ? j - 8 : 0, t, ct);
+#pragma unroll
+      for (int u = 3; u >= 0; u--) {
+        double q = v[u][5];
+        q -= c[u][0] * w3;
+        q -= c[u][1] * w2;
+        q -= c[u][2] * w1;
+        ok = ok && mf_in_range(q);
+        const double x = mf_div(q, v[u][4], v[u][3]);
+        ra[6 * (size_t)(j - 4 + u) + 5] = x;
+        w3 = w2, w2 = w1, w1 = x;
       }
-      const double xj = s / dj;
-      x[j] = xj;
-      w3 = w2, w2 = w1, w1 = xj;
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+#pragma unroll
+        for (int e = 3; e < 6; e++) v[u][e] = t[u][e];
+#pragma unroll
+        for (int e = 0; e < 3; e++) c[u][e] = ct[u][e];
+      }
     }
   }
-  __syncthreads();
-  for (uint32_t i = threadIdx.x; i < nr; i += 64)
-    m.next[m.mem[r0 + i]] = (double)flush_hd((float)x[i]);
+  mf_sync();
+  if (!__all(ok)) return false;
+  for (uint32_t i = lane; i < nr; i += 64)
+    m.next[m.mem[r0 + i]] = (double)flush_hd((float)ra[6 * (size_t)i + 5]);
+  return true;
 }
 
 // MergedFaces::add_pml (conformal.rs:2582-2638): a thread per term, T and
@@ -2511,54 +2558,46 @@ __global__ void __launch_bounds__(256) mf_pml_add(DevMerged m) {
   m.circ[g] = c;
 }
 
-// The update of the reduced currents: a wave per block of `list`, then (in
-// the launch with the merge groups) a lane per merge group. The block's lanes stage its factor in LDS and form the
-// right-hand sides; lane 0 runs the serial substitutions on LDS, the last
-// solved value kept in a register. The backward substitution goes column by
-// column (x_j = (y_j - sum over k > j, decreasing, of L_kj x_k) / L_jj), the
-// very operations of the row-by-row form in the same order. A block whose
-// image exceeds lds_bytes is solved in the global scratch row by row.
-__global__ void __launch_bounds__(64) mf_advance(DevMerged m, const uint32_t *__restrict__ list,
-                                                 int count, int lds_bytes) {
-  extern __shared__ double xs[];
-  if ((int)blockIdx.x >= count) {
-    const int q = ((int)blockIdx.x - count) * 64 + (int)threadIdx.x;
-    if (q < m.ns) mf_scalar(m, q, m.cur, m.circ, m.next);
-    return;
-  }
-  const uint32_t b = list[blockIdx.x] & 0x7fffffffu;
+// The update of one block of reduced currents by a wave (its lanes 0..63).
+// The lanes stage the block's factor in LDS and form the right-hand sides;
+// lane 0 runs the serial substitutions on LDS, the last solved value kept in
+// a register. The backward substitution goes column by column (x_j = (y_j -
+// sum over k > j, decreasing, of L_kj x_k) / L_jj), the very operations of
+// the row-by-row form in the same order. A block whose image exceeds
+// lds_bytes is solved in the global scratch row by row.
+__device__ __forceinline__ void mf_block(const DevMerged &m, uint32_t tag, double *xs,
+                                         int lds_bytes, uint32_t lane) {
+  const uint32_t b = tag & 0x7fffffffu;
   const uint32_t r0 = m.bs[b], nr = m.bs[b + 1] - r0;
-  if (list[blockIdx.x] >> 31) {
-    mf_narrow(m, r0, nr, xs);
-    return;
-  }
+  const bool narrow = tag >> 31;
+  if (narrow && mf_narrow(m, r0, nr, xs, lane)) return;
   const uint64_t e0 = m.eo[r0], nev = m.eo[r0 + nr] - e0;
   const uint32_t c0 = m.cs[r0], ncol = m.cs[r0 + nr] - c0;
-  if (mf_lds_need(nr, nev, ncol) > (size_t)lds_bytes) {
+  if (narrow || mf_lds_need(nr, nev, ncol) > (size_t)lds_bytes) {
     double *x = m.x + r0;
-    for (uint32_t i = threadIdx.x; i < nr; i += 64) x[i] = mf_rhs(m, r0, i, m.cur, m.circ);
-    __syncthreads();
-    if (threadIdx.x == 0) mf_solve(m, r0, nr, x);
-    __syncthreads();
-    for (uint32_t i = threadIdx.x; i < nr; i += 64)
+    for (uint32_t i = lane; i < nr; i += 64) x[i] = mf_rhs(m, r0, i, m.cur, m.circ);
+    mf_sync();
+    if (lane == 0) mf_solve(m, r0, nr, x);
+    mf_sync();
+    for (uint32_t i = lane; i < nr; i += 64)
       m.next[m.mem[r0 + i]] = (double)flush_hd((float)x[i]);
     return;
   }
   double *x = xs, *env = xs + nr, *cv = env + nev;
   uint32_t *ef = (uint32_t *)(cv + ncol), *eo = ef + nr, *cs = eo + nr + 1, *ck = cs + nr + 1;
-  for (uint32_t i = threadIdx.x; i < nr; i += 64) ef[i] = m.ef[r0 + i];
-  for (uint32_t i = threadIdx.x; i <= nr; i += 64) {
+  for (uint32_t i = lane; i < nr; i += 64) ef[i] = m.ef[r0 + i];
+  for (uint32_t i = lane; i <= nr; i += 64) {
     eo[i] = (uint32_t)(m.eo[r0 + i] - e0);
     cs[i] = m.cs[r0 + i] - c0;
   }
-  for (uint64_t e = threadIdx.x; e < nev; e += 64) env[e] = m.ev[e0 + e];
-  for (uint32_t e = threadIdx.x; e < ncol; e += 64) {
+  for (uint64_t e = lane; e < nev; e += 64) env[e] = m.ev[e0 + e];
+  for (uint32_t e = lane; e < ncol; e += 64) {
     cv[e] = m.cv[c0 + e];
     ck[e] = m.cr[c0 + e];
   }
-  for (uint32_t i = threadIdx.x; i < nr; i += 64) x[i] = mf_rhs(m, r0, i, m.cur, m.circ);
-  __syncthreads();
-  if (threadIdx.x == 0) {
+  for (uint32_t i = lane; i < nr; i += 64) x[i] = mf_rhs(m, r0, i, m.cur, m.circ);
+  mf_sync();
+  if (lane == 0) {
     double xp = 0.0;
     for (uint32_t i = 0; i < nr; i++) {
       const uint32_t f = ef[i];
@@ -2583,9 +2622,33 @@ __global__ void __launch_bounds__(64) mf_advance(DevMerged m, const uint32_t *__
       x[j] = xp;
     }
   }
-  __syncthreads();
-  for (uint32_t i = threadIdx.x; i < nr; i += 64)
+  mf_sync();
+  for (uint32_t i = lane; i < nr; i += 64)
     m.next[m.mem[r0 + i]] = (double)flush_hd((float)x[i]);
+}
+
+// Every block and merge group: a wave per block, the large ones (a long
+// chain each) first in thread blocks of their own with the whole LDS, then
+// four small ones per thread block, then a lane per merge group. (One launch
+// after the other took the sum of both chains.)
+__global__ void __launch_bounds__(256) mf_advance(DevMerged m, const uint32_t *__restrict__ big,
+                                                  int nbig, int lds_big,
+                                                  const uint32_t *__restrict__ small, int nsmall,
+                                                  int lds_small) {
+  extern __shared__ double xs[];
+  const uint32_t lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if ((int)blockIdx.x < nbig) {
+    if (wv == 0) mf_block(m, big[blockIdx.x], xs, lds_big, lane);
+    return;
+  }
+  const int q = ((int)blockIdx.x - nbig) * 4 + wv;
+  if (q < nsmall) {
+    mf_block(m, small[q], xs + (size_t)wv * (lds_small / 8), lds_small, lane);
+    return;
+  }
+  const int g = (q - nsmall) * 64 + (int)lane;
+  if (g < m.ns) mf_scalar(m, g, m.cur, m.circ, m.next);
 }
 
 // MergedFaces::post_h, the rest (conformal.rs:2662-2671): g = g', and every
@@ -4172,6 +4235,15 @@ int launch_pw(ems_gpu *h, const HostOp &o, const Fields &f, int stage) {
 // update on the side stream); stage 0, at the operator's place in the mid
 // gap, writes the driven faces' currents; stage 1 the circulations of the
 // energy look-ahead in the post-E gap.
+void launch_mf_advance(const HostOp &o, const DevMerged &m, hipStream_t st) {
+  const int waves = o.mf_nsmall + (m.ns + 63) / 64, nb = o.mf_nbig + (waves + 3) / 4;
+  if (nb)
+    hipLaunchKernelGGL(mf_advance, dim3(nb), dim3(256),
+                       (size_t)std::max(o.mf_lds_big, 4 * o.mf_lds_small), st, m,
+                       (const uint32_t *)o.mf_big, o.mf_nbig, o.mf_lds_big,
+                       (const uint32_t *)o.mf_small, o.mf_nsmall, o.mf_lds_small);
+}
+
 int launch_merged(ems_gpu *h, const HostOp &o, const Fields &f, int stage, hipStream_t st) {
   const DevMerged &m = o.mf;
   if (stage != 0 && m.ng)
@@ -4182,15 +4254,7 @@ int launch_merged(ems_gpu *h, const HostOp &o, const Fields &f, int stage, hipSt
     hipLaunchKernelGGL(mf_pml_add, dim3((m.ng + 255) / 256), dim3(256), 0, st, m);
   }
   if (stage == 2) {
-    // small blocks (and the merge groups) with a small LDS image, so that
-    // many waves share a CU; then the large blocks
-    const int na = o.mf_nsmall + (m.ns + 63) / 64;
-    if (na)
-      hipLaunchKernelGGL(mf_advance, dim3(na), dim3(64), (size_t)o.mf_lds_small, st, m,
-                         (const uint32_t *)o.mf_small, o.mf_nsmall, o.mf_lds_small);
-    if (o.mf_nbig)
-      hipLaunchKernelGGL(mf_advance, dim3(o.mf_nbig), dim3(64), (size_t)o.mf_lds_big, st, m,
-                         (const uint32_t *)o.mf_big, o.mf_nbig, o.mf_lds_big);
+    launch_mf_advance(o, m, st);
   }
   if (stage == 0) {
     const int nd = std::max(m.nf, m.ng);
@@ -5854,7 +5918,7 @@ int ems_gpu_add_merged(ems_gpu *h, const ems_merged_desc *d, int *id) {
     CK(h, hipEventCreateWithFlags(&h->ev_join, hipEventDisableTiming));
   }
   o.mf_nsmall = (int)small.size(), o.mf_nbig = (int)big.size();
-  o.mf_lds_small = (int)lds_small, o.mf_lds_big = (int)lds_big;
+  o.mf_lds_small = (int)((lds_small + 15) / 16 * 16), o.mf_lds_big = (int)lds_big;
   h->ops.push_back(o);
   h->ops_dirty = true;
   if (id) *id = (int)h->ops.size() - 1;
@@ -6011,13 +6075,7 @@ static int ops_energy_enqueue(ems_gpu *h) {
       int rc = merged_circ_now(h, o);
       if (rc) return rc;
       const DevMerged &m = o.mf;
-      const int na = o.mf_nsmall + (m.ns + 63) / 64;
-      if (na)
-        hipLaunchKernelGGL(mf_advance, dim3(na), dim3(64), (size_t)o.mf_lds_small, h->stream, m,
-                           (const uint32_t *)o.mf_small, o.mf_nsmall, o.mf_lds_small);
-      if (o.mf_nbig)
-        hipLaunchKernelGGL(mf_advance, dim3(o.mf_nbig), dim3(64), (size_t)o.mf_lds_big, h->stream,
-                           m, (const uint32_t *)o.mf_big, o.mf_nbig, o.mf_lds_big);
+      launch_mf_advance(o, m, h->stream);
       const int nr = (int)o.mfh->mem.size(), ng = (int)o.mfh->l.size();
       const uint32_t *row0 = o.d_erow0, *mrs = row0 + nr, *mcol = mrs + nr + 1;
       hipLaunchKernelGGL(mf_energy_terms, dim3((unsigned)((o.n_et + 255) / 256)), dim3(256), 0,
