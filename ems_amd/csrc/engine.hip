@@ -1922,42 +1922,90 @@ __global__ void __launch_bounds__(256) mur_corners(Fields f, DevMur m, const uin
 // cb = dt/((A/l)(1 + a_p)), da and db likewise), so the H and E updates
 // leave the flux increment t in the field. Edges are grouped by side and
 // axis (off[g] is the first edge of group g = 3 side + axis: E x, y, z,
-// then H x, y, z); every edge is independent of the others.
+// then H x, y, z), each group by node; every edge is independent of the
+// others.
+constexpr int UPML_RUN = 1024;  // edges per block of upml_apply
+struct UpmlChunk {
+  uint64_t base;    // first node
+  int q0, cnt, g;   // its edges: up to UPML_RUN of group g
+};
 struct DevUpml {
   int ne, nh;
   int off[7];
-  const uint64_t *idx;  // node index per edge
-  const float4 *co;     // (1-a_p)/(1+a_p), (1-a_q)/(1+a_q), (1+a_a)/((1+a_q)m), (1-a_a)/((1+a_q)m)
-  float2 *fv;           // flux F, start value v
+  int chunks[2];           // per side
+  const UpmlChunk *chunk;  // E side's, then H side's
+  const uint64_t *idx;     // node index per edge
+  const uint32_t *rel;     // the same less the chunk's base
+  // (1-a_p)/(1+a_p), (1-a_q)/(1+a_q), (1+a_a)/((1+a_q)m), (1-a_a)/((1+a_q)m):
+  // the distinct ones by code, or with no codes one per edge
+  const float4 *co;
+  const uint16_t *code;
+  float *flux, *val;  // flux F, start value v
 };
+__device__ __forceinline__ float4 upml_co(const DevUpml &m, int q) {
+  return m.co[m.code ? (int)m.code[q] : q];
+}
 
-__device__ __forceinline__ float *pick_i(const Fields &f, int a) {
-  return a == 0 ? f.i[0] : (a == 1 ? f.i[1] : f.i[2]);
+// A group's field.
+__device__ __forceinline__ float *pick6(const Fields &f, int g) {
+  float *x = f.u[0];
+  x = g == 1 ? f.u[1] : x;
+  x = g == 2 ? f.u[2] : x;
+  x = g == 3 ? f.i[0] : x;
+  x = g == 4 ? f.i[1] : x;
+  x = g == 5 ? f.i[2] : x;
+  return x;
 }
 
 // Parts::post_h_slab / post_e_slab (upml.rs:442-470). stage 0 (after the H
 // update): E edges take v from u (Run::refresh, :391-400), H edges complete
-// (Run::apply, :404-426); stage 1 (after the E update) the other way round.
-__global__ void __launch_bounds__(256) upml_stage(Fields f, DevUpml m, int stage) {
-  const int q = blockIdx.x * 256 + threadIdx.x;
-  if (q >= m.ne + m.nh) return;
-  int g = 0;
-  while (g < 5 && q >= m.off[g + 1]) g++;
-  const bool eside = g < 3;
-  const int a = eside ? g : g - 3;
-  GAS float *x = (GAS float *)(eside ? pick_u(f, a) : pick_i(f, a));
-  const uint64_t n = m.idx[q];
-  float2 s = m.fv[q];
-  if (eside == (stage == 0)) {
-    s.y = x[n];
-  } else {
-    const float4 c = m.co[q];
-    const float f1 = flush(flush(c.x * s.x) + x[n]);
-    const float v = flush(flush(flush(c.y * s.y) - flush(c.w * s.x)) + flush(c.z * f1));
-    s.x = f1, s.y = v;
-    x[n] = v;
+// (Run::apply, :404-426); stage 1 (after the E update) the other way round,
+// the H edges' refresh only where an operator may have changed i since they
+// completed (else v is what they hold). A block per chunk: `na` chunks from
+// a0 complete, then those from r0 refresh.
+//
+// Bound by the layer's bytes, per edge and step 4 of node, 2 of code, 8 of
+// flux, 8 of value and 8 of field to complete, 12 to refresh (with 64-bit
+// nodes, a float4 of coefficients and flux and value rewritten by both 48
+// and 28). 141 x 112 x 90 nodes, eight layers on every face, 3.2 M edges:
+// 2 x 12.0 us a step, before 2 x 41. Four edges per thread keep that many
+// gathers in flight.
+template <bool CODED>
+__global__ void __launch_bounds__(256) upml_stage(Fields f, DevUpml m, int na, int a0, int r0) {
+  const int blk = (int)blockIdx.x;
+  const bool apply = blk < na;
+  const int ck = apply ? a0 + blk : r0 + (blk - na);
+  const UpmlChunk *cp = m.chunk + ck;
+  const int q0 = cp->q0, cnt = cp->cnt;
+  GAS float *x = (GAS float *)pick6(f, cp->g) + cp->base;
+  constexpr int U = UPML_RUN / 256;
+  uint32_t at[U], ci[U];
+  float t[U], fl[U], v0[U];
+  float4 c[U];
+#pragma unroll
+  for (int s = 0; s < U; s++) {
+    const int q = q0 + min((int)threadIdx.x + 256 * s, cnt - 1);
+    at[s] = m.rel[q];
+    if (!apply) continue;
+    ci[s] = CODED ? m.code[q] : (uint32_t)q;
+    fl[s] = m.flux[q], v0[s] = m.val[q];
   }
-  m.fv[q] = s;
+#pragma unroll
+  for (int s = 0; s < U; s++) {
+    t[s] = x[at[s]];
+    if (apply) c[s] = m.co[ci[s]];
+  }
+#pragma unroll
+  for (int s = 0; s < U; s++) {
+    const int r = (int)threadIdx.x + 256 * s;
+    float v = t[s];
+    if (apply) {
+      const float f1 = flush(flush(c[s].x * fl[s]) + t[s]);
+      v = flush(flush(flush(c[s].y * v0[s]) - flush(c[s].w * fl[s])) + flush(c[s].z * f1));
+      if (r < cnt) m.flux[q0 + r] = f1, x[at[s]] = v;
+    }
+    if (r < cnt) m.val[q0 + r] = v;
+  }
 }
 
 __device__ __forceinline__ float op_amp(const DevOp &o, uint64_t n) {
@@ -3163,59 +3211,78 @@ __global__ void __launch_bounds__(256) energy_planes(int nx, int ny, const doubl
 // (component, plane) mu0 sum (v^2 - inc^2) over its edges in index order,
 // inc the kernel's flux increment evaluated in the Paired order as written
 // there, v the completed layer value; added to the plane in component
-// order. A wave per plane, the terms a round at a time into LDS, lane 0
-// adding them in order. hplane[c (nx + 1) + gi]: the plane's first H edge
-// of component c (device order: by component, then node index).
-__global__ void __launch_bounds__(256) upml_energy_planes(Fields f, Lanes L, DevUpml m,
+// order. hplane[c (nx + 1) + gi]: the plane's first H edge of component c
+// (device order: by component, then node index).
+//
+// A block per plane. Waves 0 to 2 add one component each, in order, from
+// LDS; the other five compute the next round's terms meanwhile (two per
+// thread and component, so that a round's loads overlap). Bound by the
+// additions of the fullest plane's longest run, one after the other: 141 x
+// 112 x 90 nodes 120 us (a wave per plane doing both in turn for the three
+// components: 805).
+__device__ __forceinline__ double upml_term(const Fields &f, const Lanes &L, const DevUpml &m,
+                                            int comp, int q, int gi, int ny, int nz) {
+  const size_t plane = (size_t)ny * nz;
+  const size_t idx = m.idx[q], o = idx - (size_t)gi * plane;
+  const int j = (int)(o / nz), k = (int)(o - (size_t)j * nz);
+  const float *ux = f.u[0], *uy = f.u[1], *uz = f.u[2];
+  float c;
+  if (comp == 0)
+    c = (uz[idx + nz] - uz[idx]) - (uy[idx + 1] - uy[idx]);
+  else if (comp == 1)
+    c = (ux[idx + 1] - ux[idx]) - (uz[idx + plane] - uz[idx]);
+  else
+    c = (uy[idx + plane] - uy[idx]) - (ux[idx + nz] - ux[idx]);
+  const float db = coef(pick_lane(L, 9 + comp), (size_t)gi * ny + j, k, nz, idx);
+  const float F = m.flux[q], V = m.val[q];
+  const float4 co = upml_co(m, q);
+  const float inc = flush(0.0f * V - db * c);
+  const float f1 = flush(flush(co.x * F) + inc);
+  const float v = flush(flush(flush(co.y * V) - flush(co.w * F)) + flush(co.z * f1));
+  return (double)v * (double)v - (double)inc * (double)inc;
+}
+
+__global__ void __launch_bounds__(512) upml_energy_planes(Fields f, Lanes L, DevUpml m,
                                                           const uint32_t *hplane, int nx, int ny,
                                                           int nz, double *planes) {
-  __shared__ double buf[4][256];
-  const int wv = threadIdx.x >> 6, t = threadIdx.x & 63;
-  const int gi = (int)blockIdx.x * 4 + wv;
-  if (gi >= nx) return;  // uniform per wave
-  const size_t plane = (size_t)ny * nz;
-  double *b = buf[wv];
-  double pv = t == 0 ? planes[gi] : 0.0;
-  for (int comp = 0; comp < 3; comp++) {
-    const uint32_t r0 = hplane[comp * (nx + 1) + gi], r1 = hplane[comp * (nx + 1) + gi + 1];
-    if (r0 == r1) continue;  // no run
-    const Lane ldb = pick_lane(L, 9 + comp);
-    double sum = 0.0;
-    for (uint32_t q0 = r0; q0 < r1; q0 += 256) {
+  constexpr int TERMS = 320 * 2;  // per component and round
+  __shared__ double buf[2][3][TERMS], sums[3];
+  const int gi = (int)blockIdx.x, wv = threadIdx.x >> 6, p = (int)threadIdx.x - 192;
+  int r0[3], n[3], rounds = 0;
 #pragma unroll
-      for (int s = 0; s < 4; s++) {
-        const uint32_t q = q0 + 64 * s + t;
-        double term = 0.0;
-        if (q < r1) {
-          const size_t idx = m.idx[q], o = idx - (size_t)gi * plane;
-          const int j = (int)(o / nz), k = (int)(o - (size_t)j * nz);
-          const float *ux = f.u[0], *uy = f.u[1], *uz = f.u[2];
-          float c;
-          if (comp == 0)
-            c = (uz[idx + nz] - uz[idx]) - (uy[idx + 1] - uy[idx]);
-          else if (comp == 1)
-            c = (ux[idx + 1] - ux[idx]) - (uz[idx + plane] - uz[idx]);
-          else
-            c = (uy[idx + plane] - uy[idx]) - (ux[idx + nz] - ux[idx]);
-          const float db = coef(ldb, (size_t)gi * ny + j, k, nz, idx);
-          const float2 st = m.fv[q];
-          const float4 co = m.co[q];
-          const float inc = flush(0.0f * st.y - db * c);
-          const float f1 = flush(flush(co.x * st.x) + inc);
-          const float v = flush(flush(flush(co.y * st.y) - flush(co.w * st.x)) + flush(co.z * f1));
-          term = (double)v * (double)v - (double)inc * (double)inc;
-        }
-        b[64 * s + t] = term;
-      }
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      if (t == 0) sum = chain_add(sum, b, 0, (int)min(256u, r1 - q0), 1);
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-    }
-    if (t == 0) pv += MU0_D * sum;
+  for (int c = 0; c < 3; c++) {
+    r0[c] = (int)hplane[c * (nx + 1) + gi];
+    n[c] = (int)hplane[c * (nx + 1) + gi + 1] - r0[c];
+    rounds = max(rounds, (n[c] + TERMS - 1) / TERMS);
   }
-  if (t == 0) planes[gi] = pv;
+  auto fill = [&](int round) {
+#pragma unroll
+    for (int c = 0; c < 3; c++)
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+        const int e = round * TERMS + s * 320 + p;
+        if (e < n[c]) buf[round & 1][c][s * 320 + p] = upml_term(f, L, m, c, r0[c] + e, gi, ny, nz);
+      }
+  };
+  if (p >= 0 && rounds > 0) fill(0);
+  double sum = 0.0;
+  for (int round = 0; round < rounds; round++) {
+    __syncthreads();
+    if (p >= 0) {
+      if (round + 1 < rounds) fill(round + 1);
+    } else if ((threadIdx.x & 63) == 0) {
+      const int left = (wv == 0 ? n[0] : (wv == 1 ? n[1] : n[2])) - round * TERMS;
+      if (left > 0) sum = chain_add(sum, buf[round & 1][wv], 0, min(left, TERMS), 1);
+    }
+  }
+  if (wv < 3 && (threadIdx.x & 63) == 0) sums[wv] = sum;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double pv = planes[gi];
+    for (int c = 0; c < 3; c++)
+      if (n[c] > 0) pv += MU0_D * sums[c];
+    planes[gi] = pv;
+  }
 }
 
 // The kernel's look-ahead i^{n+1/2} of listed dual edges (dump.rs:1830-1845),
@@ -3246,10 +3313,10 @@ __global__ void __launch_bounds__(64) lookahead_edges(Fields f, Lanes L, int n, 
       if (m.idx[mid] < o) lo = mid + 1; else hi = mid;
     }
     if (lo < m.off[4 + c] && m.idx[lo] == o) {
-      const float2 s = m.fv[lo];
-      const float4 co = m.co[lo];
-      const float f1 = flush(flush(co.x * s.x) + k);
-      k = flush(flush(flush(co.y * s.y) - flush(co.w * s.x)) + flush(co.z * f1));
+      const float F = m.flux[lo];
+      const float4 co = upml_co(m, lo);
+      const float f1 = flush(flush(co.x * F) + k);
+      k = flush(flush(flush(co.y * m.val[lo]) - flush(co.w * F)) + flush(co.z * f1));
     }
   }
   out[q] = k;
@@ -3600,6 +3667,17 @@ bool has_merged(const ems_gpu *h) {
 bool has_upml(const ems_gpu *h) {
   for (auto &o : h->ops)
     if (o.type == OP_UPML) return true;
+  return false;
+}
+
+// Whether an operator may change i between the H-side slab corrections and
+// the E update: all but E sources, probes, lumped elements and PML layers.
+bool h_changed_mid(const ems_gpu *h) {
+  for (auto &o : h->ops) {
+    if (o.type == OP_PROBE || o.type == OP_LUMPED || o.type == OP_UPML) continue;
+    if (o.type == OP_SOURCE && (o.kind == 0 || o.kind == 1)) continue;
+    return true;
+  }
   return false;
 }
 
@@ -4398,10 +4476,14 @@ int launch_mur(ems_gpu *h, const Fields &f, int stage) {
 int launch_upml(ems_gpu *h, const Fields &f, int stage) {
   for (auto &o : h->ops) {
     if (o.type != OP_UPML) continue;
-    const int n = o.upml.ne + o.upml.nh;
-    if (n)
-      hipLaunchKernelGGL(upml_stage, dim3((n + 255) / 256), dim3(256), 0, h->stream, f, o.upml,
-                         stage);
+    const DevUpml &m = o.upml;
+    const int ce = m.chunks[0], ch = m.chunks[1];
+    const int na = stage ? ce : ch, nr = stage ? (h_changed_mid(h) ? ch : 0) : ce;
+    const int a0 = stage ? 0 : ce, r0 = stage ? ce : 0;
+    const dim3 g((unsigned)(na + nr)), b(256);
+    if (!g.x) continue;
+    if (m.code) hipLaunchKernelGGL(upml_stage<true>, g, b, 0, h->stream, f, m, na, a0, r0);
+    else hipLaunchKernelGGL(upml_stage<false>, g, b, 0, h->stream, f, m, na, a0, r0);
     CK(h, hipGetLastError());
   }
   return 0;
@@ -4792,8 +4874,8 @@ int energy_kernels_t(ems_gpu *h, double *rowsum, double *chains, double *planes,
   if (MEAS)
     for (auto &o : h->ops)
       if (o.type == OP_UPML && o.upml.nh) {
-        hipLaunchKernelGGL(upml_energy_planes, gp, dim3(256), 0, h->stream, f, lanes_arg(h), o.upml,
-                           (const uint32_t *)o.d_hplane, nx, ny, nz, planes);
+        hipLaunchKernelGGL(upml_energy_planes, dim3((unsigned)nx), dim3(512), 0, h->stream, f,
+                           lanes_arg(h), o.upml, (const uint32_t *)o.d_hplane, nx, ny, nz, planes);
         CK(h, hipGetLastError());
       }
   hipLaunchKernelGGL(energy_combine<MEAS>, dim3(1), dim3(64), 0, h->stream, nx, planes, h->dt,
@@ -5167,10 +5249,9 @@ int ems_gpu_add_upml(ems_gpu *h, const ems_upml_desc *d, int *id) {
   const float *cf[2] = {d->e_coef, d->h_coef};
   for (int s = 0; s < 2; s++)
     if (cnt[s] && (!ax[s] || !nd[s] || !cf[s])) return fail(h, EMS_E_INVALID, "PML arrays");
-  const uint64_t N = (uint64_t)h->n[0] * h->n[1] * h->n[2];
   // Grouped by (side, axis), each group in the given order.
   std::vector<int> order[6];
-  std::vector<uint64_t> flat[2], keys;
+  std::vector<uint64_t> flat[2];
   for (int s = 0; s < 2; s++) {
     flat[s].resize(cnt[s]);
     for (int q = 0; q < cnt[s]; q++) {
@@ -5182,16 +5263,18 @@ int ems_gpu_add_upml(ems_gpu *h, const ems_upml_desc *d, int *id) {
           return fail(h, EMS_E_INVALID, "PML coefficient not finite");
       flat[s][q] = ((uint64_t)p[0] * h->n[1] + p[1]) * h->n[2] + p[2];
       order[3 * s + a].push_back(q);
-      keys.push_back((uint64_t)(3 * s + a) * N + flat[s][q]);
     }
   }
-  std::sort(keys.begin(), keys.end());
-  if (std::adjacent_find(keys.begin(), keys.end()) != keys.end())
-    return fail(h, EMS_E_INVALID, "PML edge listed twice");
   // each group by node index (the layer runs' order, upml.rs:290-330)
-  for (int g = 0; g < 6; g++)
-    std::stable_sort(order[g].begin(), order[g].end(),
-                     [&](int x, int y) { return flat[g / 3][x] < flat[g / 3][y]; });
+  for (int g = 0; g < 6; g++) {
+    const std::vector<uint64_t> &fl = flat[g / 3];
+    const auto less = [&](int x, int y) { return fl[x] < fl[y]; };
+    if (!std::is_sorted(order[g].begin(), order[g].end(), less))
+      std::stable_sort(order[g].begin(), order[g].end(), less);
+    for (size_t r = 1; r < order[g].size(); r++)
+      if (fl[order[g][r]] == fl[order[g][r - 1]])
+        return fail(h, EMS_E_INVALID, "PML edge listed twice");
+  }
   HostOp o;
   o.type = OP_UPML;
   DevUpml &m = o.upml;
@@ -5210,15 +5293,67 @@ int ems_gpu_add_upml(ems_gpu *h, const ems_upml_desc *d, int *id) {
     }
     m.off[g + 1] = (int)idx.size();
   }
+  // Blocks of up to UPML_RUN edges of one group, nodes relative to the first.
+  std::vector<UpmlChunk> chunk;
+  std::vector<uint32_t> rel(n);
+  for (int g = 0; g < 6; g++) {
+    for (int q = m.off[g]; q < m.off[g + 1]; q++) {
+      if (q == m.off[g] || chunk.back().cnt == UPML_RUN ||
+          idx[q] - chunk.back().base > 0xFFFFFFFFull)
+        chunk.push_back({idx[q], q, 0, g}), m.chunks[g / 3]++;
+      rel[q] = (uint32_t)(idx[q] - chunk.back().base);
+      chunk.back().cnt++;
+    }
+  }
+  // The distinct coefficients (a few per depth, side and material; most
+  // edges repeat the one before or the one a row before), unless 16 bits
+  // cannot number them.
+  std::vector<uint16_t> code(n);
+  std::vector<float4> table;
+  {
+    size_t cap = 64;  // (open addressing: place of a coefficient's code + 1)
+    while (cap < 2 * std::min<size_t>(n, 65537)) cap *= 2;
+    std::vector<uint32_t> at(cap);
+    bool fits = true;
+    for (size_t q = 0; q < n && fits; q++) {
+      if (q && !std::memcmp(&co[q], &co[q - 1], sizeof(float4))) {
+        code[q] = code[q - 1];
+        continue;
+      }
+      uint32_t k[4];
+      std::memcpy(k, &co[q], sizeof k);
+      uint64_t x = 0;
+      for (uint32_t w : k) x = (x ^ w) * 0x9E3779B97F4A7C15ull, x ^= x >> 29;
+      size_t r = x & (cap - 1);
+      while (at[r] && std::memcmp(&table[at[r] - 1], k, sizeof k)) r = (r + 1) & (cap - 1);
+      if (!at[r]) table.push_back(co[q]), at[r] = (uint32_t)table.size();
+      fits = table.size() <= 65536;
+      code[q] = (uint16_t)(at[r] - 1);
+    }
+    if (!fits) code.clear(), table = co;
+  }
   int rc;
   void *p = nullptr;
-  if ((rc = upload(h, &p, idx.data(), n * sizeof(uint64_t)))) return rc;
-  o.mem.push_back(p), m.idx = (const uint64_t *)p;
-  if ((rc = upload(h, &p, co.data(), n * sizeof(float4)))) return rc;
-  o.mem.push_back(p), m.co = (const float4 *)p;
-  std::vector<float2> zero(n, make_float2(0.0f, 0.0f));
-  if ((rc = upload(h, &p, zero.data(), n * sizeof(float2)))) return rc;
-  o.mem.push_back(p), m.fv = (float2 *)p;
+  auto up = [&](const auto &v) -> int {
+    const int e = upload(h, &p, v.data(), v.size() * sizeof(v[0]));
+    if (!e) o.mem.push_back(p);
+    return e;
+  };
+  if ((rc = up(idx))) return rc;
+  m.idx = (const uint64_t *)p;
+  if ((rc = up(rel))) return rc;
+  m.rel = (const uint32_t *)p;
+  if ((rc = up(chunk))) return rc;
+  m.chunk = (const UpmlChunk *)p;
+  if ((rc = up(table))) return rc;
+  m.co = (const float4 *)p;
+  if (!code.empty()) {
+    if ((rc = up(code))) return rc;
+    m.code = (const uint16_t *)p;
+  }
+  const std::vector<float> zero(2 * n, 0.0f);
+  if ((rc = up(zero))) return rc;
+  m.flux = (float *)p, m.val = m.flux + n;
   // The caller's order of each side, for ems_gpu_upml_state.
   std::vector<uint32_t> pos(n);
   for (int g = 0; g < 6; g++)
@@ -5251,13 +5386,13 @@ int ems_gpu_upml_state(ems_gpu *h, int id, int side, float *flux, float *value) 
   const int cnt = side ? o.upml.nh : o.upml.ne;
   if (cnt && (!flux || !value)) return EMS_E_INVALID;
   const size_t n = (size_t)o.upml.ne + o.upml.nh;
-  std::vector<float2> fv(n);
+  std::vector<float> fv(2 * n);
   CK(h, hipStreamSynchronize(h->stream));
-  if (n) CK(h, hipMemcpy(fv.data(), o.upml.fv, n * sizeof(float2), hipMemcpyDeviceToHost));
+  if (n) CK(h, hipMemcpy(fv.data(), o.upml.flux, 2 * n * sizeof(float), hipMemcpyDeviceToHost));
   const size_t base = side ? o.upml.ne : 0;
   for (int q = 0; q < cnt; q++) {
-    const float2 s = fv[o.upml_pos[base + q]];
-    flux[q] = s.x, value[q] = s.y;
+    const size_t e = o.upml_pos[base + q];
+    flux[q] = fv[e], value[q] = fv[n + e];
   }
   return EMS_OK;
 }

@@ -234,3 +234,34 @@ def test_reduced_current_block_paths():
         assert np.float64(wg).tobytes() == np.float64(wo).tobytes(), (n, wg, wo)
     same_fields(g, o)
     assert np.abs(pg.currents()[0]).max() > 0.0
+
+
+@pytest.mark.parametrize("sizes", [[-1, -3, -4, -5], [-61, -300]], ids=str)
+@pytest.mark.parametrize("scale", [1.0, 1e-54], ids=["in_range", "out_of_range"])
+def test_narrow_blocks(sizes, scale, monkeypatch):
+    """Tridiagonal blocks around multiples of four rows, and factors beyond
+    the range of the reciprocal's quotients (the plain substitution), bit
+    for bit."""
+    from ems_amd import merged as MF
+    factor = MF.Envelope.factor
+    monkeypatch.setattr(MF.Envelope, "factor", staticmethod(
+        lambda rows: factor([[(j, v * scale) for j, v in r] for r in rows])))
+
+    def build(kind):
+        g = E.Grid.uniform([10, 9, 8], [1e-3] * 3)
+        e = K.make(kind, g, None)
+        op = _synthetic_merged(g, e.dt, sizes)
+        e.add_operator(op)
+        rng = np.random.default_rng(11)
+        for a in range(3):
+            u = rng.standard_normal(g.nodes()) * (1.0 if scale == 1.0 else 1e-30)
+            e.set_component(0, a, u.astype(np.float32))
+        return e, op
+    (g, pg), (o, po) = build("gpu"), build("oracle")
+    for n in (1, 3, 6) if scale == 1.0 else (1,):  # (the tiny factor's second step overflows f32)
+        g.run(n)
+        o.run(n)
+        for x, y in zip(pg.currents(), po.currents()):
+            assert np.array_equal(bits(x), bits(y)), n
+    same_fields(g, o)
+    assert np.abs(pg.currents()[0][1:]).max() > 0.0

@@ -165,3 +165,61 @@ def test_edge_listed_twice_is_refused():
     with pytest.raises(E.EmsError, match="twice"):
         e.add_operator(op)
     e.close()
+
+
+@pytest.mark.parametrize("edges", [1, 1023, 1025, None], ids=str)
+@pytest.mark.parametrize("h_source", [False, True], ids=["e_source", "h_source"])
+def test_layer_edge_counts_and_coefficients(edges, h_source):
+    """Layers of few edges per group, given in no order, around the edges one
+    block takes, and layers with more distinct coefficients than 16 bits number;
+    with and without an operator that changes i between the updates, and
+    fields written between runs. Fields, layer state and both energies."""
+    cells = (14, 12, 13) if edges else (39, 34, 31)
+
+    def build(kind):
+        gr = E.Grid.uniform(list(cells), [1e-3] * 3)
+        dt = E.TimeStep.courant(0.95).resolve(gr)
+        lanes = E.coefficients(gr, None, [E.FaceCondition.Pec] * 6, dt)
+        e = (E.Engine(gr, dt, lanes, curl_order=1) if kind == "gpu"
+             else OracleEngine(gr, dt, lanes, curl_order=1, threads=3))
+        rng = np.random.default_rng(5)
+        n = gr.nodes()
+        op = E.OpenEmsPml.with_materials(e, [(E.Face.XMax, 6), (E.Face.YMin, 5), (E.Face.ZMax, 5)],
+                                         1.0 + rng.random((3,) + n), 1.0 + rng.random((3,) + n))
+        if edges:
+            for side in "eh":
+                ax, nd, co = getattr(op, side)
+                pick = np.concatenate([rng.permutation(np.flatnonzero(ax == a))[:max(1, edges - 7 * a)]
+                                       for a in range(3)])
+                pick = np.sort(pick)
+                perm[side] = rng.permutation(pick.size)
+                if kind == "gpu":  # (the oracle adds the energy in the order given)
+                    pick = pick[perm[side]]
+                setattr(op, side, (ax[pick], nd[pick], co[pick]))
+        else:
+            assert len(np.unique(np.concatenate([op.e[2], op.h[2]]), axis=0)) > 65536
+        e.add_operator(op)
+        src = E.EdgeSource(E.Waveform.gaussian(2e10, 1e10))
+        if h_source:
+            src.kind(E.SourceKind.SoftH)
+        e.add_operator(src.edge(E.Axis.X, [6, 1, 6], 1e-3).edge(E.Axis.Y, [5, 5, 5], 1e-3))
+        return e, op
+    perm = {"e": slice(None), "h": slice(None)}
+    (g, gop), (o, oop) = build("gpu"), build("oracle")
+    rng = np.random.default_rng(6)
+    for n in (1, 2, 9, 40):
+        for f in (0, 1):
+            for a in range(3):
+                v = (rng.standard_normal(g.grid.nodes()) * (1e-3 if f else 1.0)).astype(np.float32)
+                g.set_component(f, a, v)
+                o.set_component(f, a, v)
+        g.run(n)
+        o.run(n)
+        same_fields(g, o)
+        for s, side in enumerate("eh"):
+            for a, b in zip(g.upml_state(gop, s), o.upml_state(oop, s)):
+                assert np.array_equal(bits(a), bits(b[perm[side]])), (n, side)
+        for a, b in ((g.energy(), o.energy()), (g.energy_openems(), o.energy_openems())):
+            assert np.float64(a).tobytes() == np.float64(b).tobytes(), n
+    g.close()
+    o.close()
