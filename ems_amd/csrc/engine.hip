@@ -14,11 +14,13 @@
 //
 // Kernels (one stream; one step = H, CPML-H slabs, mid gap, E, CPML-E slabs,
 // post-E gap), captured into HIP graphs of whole steps:
-//   h_update / e_update: one thread per in-plane node p = j*nz + k (z fastest,
-//     fully coalesced over the contiguous ny*nz plane), marching a chunk of
-//     x-planes and carrying the neighbour plane it already loaded in
-//     registers (uy, uz of plane i+1 for H; iy, iz of plane i-1 for E).
-//   cpml_slab: one thread per node of a slab box.
+//   h_update_quad / e_update_quad (default): four nodes of a z row per
+//     thread, the side's CPML slabs corrected inside.
+//   h_update / e_update: one thread per in-plane node p = j*nz + k, two
+//     x-planes each.
+//   cpml_slab: one thread per node of a slab box (irregular slab sets).
+//   step_*: H and E of a step in one launch from one buffer into the other
+//     (set schedules, the autotuner, batches).
 //   gap_mid / gap_post_e: one thread runs the serial operator hooks in
 //     registration order (they are few and must stay ordered).
 //   energy_*: the invariant as f64 chains in exactly the reference's order.
@@ -4924,14 +4926,15 @@ int run_steps(ems_gpu *h, uint64_t n) {
   if (n == 0) return 0;
   int rc = prepare(h, n);
   if (rc) return rc;
-  const int p0 = h->par;
-  if (!h->g1[p0]) {
-    for (int p = 0; p < 2; p++) {
-      if ((rc = capture(h, 1, p, &h->g1[p]))) return rc;
-      if ((rc = capture(h, h->K, p, &h->gK[p]))) return rc;
-    }
-  }
   const int flip = use_fused(h) ? 1 : 0;
+  // A graph is captured by the first run that launches it (all four of them
+  // on the first run took 0.5 ms of the first single step of a 24^3 box).
+  const uint64_t singles = n % (uint64_t)h->K;
+  if (n != singles && !h->gK[h->par])
+    if ((rc = capture(h, h->K, h->par, &h->gK[h->par]))) return rc;
+  for (int q = 0; q <= flip && (uint64_t)q < singles; q++)
+    if (!h->g1[h->par ^ q])
+      if ((rc = capture(h, 1, h->par ^ q, &h->g1[h->par ^ q]))) return rc;
   uint64_t left = n;
   while (left >= (uint64_t)h->K) {
     CK(h, hipGraphLaunch(h->gK[h->par], h->stream));
@@ -7179,13 +7182,16 @@ int ems_gpu_batch_run(ems_gpu_batch *b, const uint8_t *active, uint64_t n) {
   }
   if (act != b->active) {
     batch_drop_graphs(b);
-    for (int p = 0; p < 2; p++) {
-      if ((rc = batch_capture(b, act, 1, p, &b->g1[p]))) return rc;
-      if ((rc = batch_capture(b, act, b->K, p, &b->gK[p]))) return rc;
-    }
     b->active = act;
   }
   int p = par;
+  // (captured by the first run that launches them)
+  const uint64_t singles = n % (uint64_t)b->K;
+  if (n != singles && !b->gK[p])
+    if ((rc = batch_capture(b, act, b->K, p, &b->gK[p]))) return rc;
+  for (int q = 0; q < 2 && (uint64_t)q < singles; q++)
+    if (!b->g1[p ^ q])
+      if ((rc = batch_capture(b, act, 1, p ^ q, &b->g1[p ^ q]))) return rc;
   uint64_t left = n;
   while (left >= (uint64_t)b->K) {
     BCK(b, hipGraphLaunch(b->gK[p], b->stream));
