@@ -184,7 +184,7 @@ def sweep(args, log) -> int:
     per_step = (time.perf_counter() - tk) / 64
     byt = sum(e.traffic_model()[0] for e, a in zip(engines, act) if a)
     achieved = byt / per_step / 1e9
-    kname = "step_packed_batch" if packed else "step_fused_batch"
+    kname = "quad_batch" if packed else "step_fused_batch"
     traffic, traffic_cfg = None, None
     tpath = os.path.join(ROOT, "profiles", f"{kname}_patch_sweep_{len(models)}.json")
     if os.path.exists(tpath):
@@ -197,7 +197,7 @@ def sweep(args, log) -> int:
             "traffic_measured_at": traffic_cfg,
             "bytes_per_launch": byt, "launch_ms": round(per_step * 1e3, 4),
             "models": int(sum(act)),
-            "timing": "wall clock of synchronised batch runs (64 steps, fused and gap kernels); "
+            "timing": "wall clock of synchronised batch runs (64 steps, step and gap kernels); "
                       "counters from a run without graphs"}
     log(f"batched kernel: {per_step*1e3:.3f} ms per step over {sum(act)} models, "
         f"{achieved:.0f} GB/s algorithmic")
@@ -480,7 +480,7 @@ def main() -> int:
                    "cpml_cells": {"cpml_box": 8, "dispersive_box": 10}.get(args.workload, 0),
                    "energy_every": energy_every or None,
                    "probes": len(probes), "parallelism": "single GPU",
-                   "schedule": "unfused" if args.unfused else "fused",
+                   "schedule": "unfused" if te else "fused",
                    "mode": None if args.unfused else (tuned["mode"] if tuned else args.mode),
                    "autotune": tuned},
         "roofline": roof, "cpu_baseline": cpu,
