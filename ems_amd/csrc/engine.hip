@@ -2449,6 +2449,12 @@ __host__ __device__ __forceinline__ size_t mf_narrow_need(uint32_t nr) {
   return 72 * (size_t)((nr + 3) / 4 * 4);
 }
 
+// The largest image of a narrow block: 1024 rows (two such fit a CU's LDS).
+// Longer ones are substituted by the general code, or, with three values
+// below the diagonal, from the global scratch: a step with 963 such rows takes
+// 202 us as a narrow block and 1068 from the scratch.
+constexpr size_t MF_NARROW_LDS = 73728;
+
 // The wave's own writes (LDS and memory) before its reads after it. (Blocks
 // are solved by single waves, several of them in one thread block.)
 __device__ __forceinline__ void mf_sync() {
@@ -6039,7 +6045,7 @@ int ems_gpu_add_merged(ems_gpu *h, const ems_merged_desc *d, int *id) {
     size_t need = mf_lds_need(r1 - r0, d->env_off[r1] - d->env_off[r0],
                               d->col_start[r1] - d->col_start[r0]);
     uint32_t tag = b;
-    if (narrow && mf_narrow_need(r1 - r0) <= 65536) {
+    if (narrow && mf_narrow_need(r1 - r0) <= MF_NARROW_LDS) {
       need = mf_narrow_need(r1 - r0);
       tag |= 0x80000000u;
     }
@@ -6048,9 +6054,12 @@ int ems_gpu_add_merged(ems_gpu *h, const ems_merged_desc *d, int *id) {
       lds_small = std::max(lds_small, need);
     } else {
       big.push_back(tag);
-      if (need <= 65536) lds_big = std::max(lds_big, need);
+      if (need <= 65536 || tag >> 31) lds_big = std::max(lds_big, need);
     }
   }
+  if (lds_big > 65536)
+    CK(h, hipFuncSetAttribute((const void *)mf_advance, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)MF_NARROW_LDS));
   if ((rc = put(small.data(), small.size() * sizeof(uint32_t), (void **)&o.mf_small))) return rc;
   if ((rc = put(big.data(), big.size() * sizeof(uint32_t), (void **)&o.mf_big))) return rc;
   if (!h->side) {

@@ -6,6 +6,7 @@ sliver face merged and interpolated; fields, probes, reduced currents and
 energy bit for bit. Engines with reduced currents run the unfused
 schedule whatever is asked."""
 import math
+import time
 
 import numpy as np
 import pytest
@@ -162,12 +163,13 @@ def test_conformal_rod_in_cpml_box():
     same_fields(g, o)
 
 
-def _synthetic_merged(grid, dt, sizes, seed=3):
+def _synthetic_merged(grid, dt, sizes, seed=3, band=1):
     """A MergedFaces operator built by hand: one merge group, then one block
     per entry of `sizes` with a full (dense) factor, so that the device runs
     its general LDS path (a small dense block), its global-scratch path (a
-    block whose image exceeds 64 KiB) and its narrow path (a tridiagonal
-    block); circulation terms on random edges, driven faces with two weights."""
+    block whose image exceeds 64 KiB) and its narrow path (a block of `band`
+    values beside the diagonal); circulation terms on random edges, driven
+    faces with two weights."""
     from ems_amd import merged as MF
     rng = np.random.default_rng(seed)
     n = grid.nodes()
@@ -190,8 +192,8 @@ def _synthetic_merged(grid, dt, sizes, seed=3):
         for i in range(m):
             row = [(i, 4.0e-9 + 1e-10 * i)]
             for j in range(m):
-                if j != i and (sz > 0 or abs(i - j) == 1):
-                    row.append((j, -1.0e-9 / m if sz > 0 else -1.0e-9))
+                if j != i and (sz > 0 or abs(i - j) <= band):
+                    row.append((j, -1.0e-9 / m if sz > 0 else -1.0e-9 / band))
             rows.append(sorted(row))
         fac = MF.Envelope.factor(rows)
         assert fac is not None
@@ -265,3 +267,47 @@ def test_narrow_blocks(sizes, scale, monkeypatch):
             assert np.array_equal(bits(x), bits(y)), n
     same_fields(g, o)
     assert np.abs(pg.currents()[0][1:]).max() > 0.0
+
+
+@pytest.mark.parametrize("rows", [907, 963, 1024, 1025])
+def test_long_narrow_blocks(rows):
+    """Blocks of three values beside the diagonal around the most rows the
+    narrow path takes, bit for bit."""
+    def build(kind):
+        g = E.Grid.uniform([10, 9, 8], [1e-3] * 3)
+        e = K.make(kind, g, None)
+        op = _synthetic_merged(g, e.dt, [-rows, 20], band=3)
+        e.add_operator(op)
+        rng = np.random.default_rng(11)
+        for a in range(3):
+            e.set_component(0, a, rng.standard_normal(g.nodes()).astype(np.float32))
+        return e, op
+    (g, pg), (o, po) = build("gpu"), build("oracle")
+    for n in (1, 3):
+        g.run(n)
+        o.run(n)
+        for x, y in zip(pg.currents(), po.currents()):
+            assert np.array_equal(bits(x), bits(y)), n
+    same_fields(g, o)
+    assert np.abs(pg.currents()[0][1:]).max() > 0.0
+
+
+def test_long_narrow_blocks_keep_their_path():
+    """A narrow block's time grows with its rows up to 1024 of them (the
+    substitution in the global scratch takes five times as long a row)."""
+    times = []
+    for rows in (480, 963, 1024):
+        g = E.Grid.uniform([10, 9, 8], [1e-3] * 3)
+        e = K.make("gpu", g, None)
+        e.add_operator(_synthetic_merged(g, e.dt, [-rows], band=3))
+        e.run(32)
+        best = math.inf
+        for _ in range(3):
+            e.synchronize()
+            t0 = time.perf_counter()
+            e.run(64)
+            e.synchronize()
+            best = min(best, time.perf_counter() - t0)
+        times.append(best / rows)
+        e.close()
+    assert times[1] < 2.5 * times[0] and times[2] < 2.5 * times[0], times
