@@ -3552,7 +3552,7 @@ struct ems_gpu {
   bool croff_wide = false;  // the pool is 4 GiB or more (only the tiled kernel addresses it)
   bool lanes_dirty = true;
   int par = 0;     // buffer holding the current state
-  int lock = 0;    // parity of the steps taken while the fused schedule was open (batches)
+  int lock = 0;    // parity of the steps but those taken on schedule 0 (batches)
   int boff = 0;    // during a batch run: par relative to the batch's
   Lane lanes[12]{};
   uint64_t lane_rows[12] = {0};
@@ -7156,7 +7156,8 @@ int ems_gpu_batch_run(ems_gpu_batch *b, const uint8_t *active, uint64_t n) {
                    "model " + std::to_string(q) +
                        " needs the unfused schedule (H source, magnetic poles, plane wave, "
                        "cut-face currents, openEMS PML layers or more than 32 CPML slabs)");
-    if (h->lock != lock) return bfail(b, EMS_E_INVALID, "models of a batch step in lockstep");
+    if (((h->step ^ b->m[act[0]]->step) & 1) && h->lock != lock)
+      return bfail(b, EMS_E_INVALID, "models of a batch step in lockstep");
     h->boff = h->par ^ par;
     boffs.push_back(h->boff);
     const int rc = prepare(h, n, false);

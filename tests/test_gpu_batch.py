@@ -145,3 +145,35 @@ def test_batch_after_single_runs():
         for f in (0, 1):
             for k in range(3):
                 assert np.array_equal(x._read(f, k).view(np.uint32), y._read(f, k).view(np.uint32))
+
+
+@pytest.mark.parametrize("packed", [False, True])
+def test_batch_takes_models_of_equal_steps_on_any_schedule(packed):
+    """Models that took the same steps, one of them unfused by choice (as the
+    autotuner may leave it), are in step; so are models an odd number of
+    unfused steps apart; models that are in step by neither count are not."""
+    ms = models()[:2]
+    (a, _), (b, _), (c, _), (d, _) = (engine(ms[q]) for q in (0, 1, 0, 1))
+    a.set_schedule(0)
+    batch = E.EngineBatch([a, b])
+    batch.set_schedule(7, 2, packed=packed)
+    a.run(3)
+    batch.run(2)
+    batch.run(2, [True, False])
+    b.run(3)
+    batch.run(18)
+    c.run(25)
+    d.run(23)
+    for x, y in ((a, c), (b, d)):
+        same_fields(x, y)
+    x, y = engine(ms[0])[0], engine(ms[1])[0]
+    x.set_schedule(0)
+    x.run(2)
+    y.run(1)
+    out = E.EngineBatch([x, y])
+    with pytest.raises(E.EmsError, match="lockstep"):
+        out.run(2)
+    out.close()
+    batch.close()
+    for e in (a, b, c, d, x, y):
+        e.close()
