@@ -182,7 +182,11 @@ def sweep(args, log) -> int:
     tk = time.perf_counter()
     b.run(64, act)
     per_step = (time.perf_counter() - tk) / 64
-    byt = sum(e.traffic_model()[0] for e, a in zip(engines, act) if a)
+    # (of one step: the quad kernels' H and E, or the fused kernel)
+    if not packed:
+        for e in engines:
+            e.set_schedule(2, tj, args.x_chunks)
+    byt = sum(sum(e.traffic_model()) for e, a in zip(engines, act) if a)
     achieved = byt / per_step / 1e9
     kname = "quad_batch" if packed else "step_fused_batch"
     traffic, traffic_cfg = None, None

@@ -3553,6 +3553,7 @@ struct ems_gpu {
   bool lanes_dirty = true;
   int par = 0;     // buffer holding the current state
   int lock = 0;    // parity of the steps but those taken on schedule 0 (batches)
+  bool counts = true;  // whether its own steps count: not once set to 0, until a batch run
   int boff = 0;    // during a batch run: par relative to the batch's
   Lane lanes[12]{};
   uint64_t lane_rows[12] = {0};
@@ -3574,8 +3575,8 @@ struct ems_gpu {
   bool ops_dirty = true, slabs_dirty = true;
   uint64_t step = 0;
   uint64_t *d_step = nullptr;
-  // until ems_gpu_set_schedule or a batch picks one, the schedule is the
-  // engine's choice (use_fused)
+  // until ems_gpu_set_schedule picks one, the schedule is the engine's
+  // choice (use_fused)
   bool auto_sched = true;
   // fused schedule and its tiling
   bool fused = true, prefetch = true, rows = false, packed = false, band = false;
@@ -3692,12 +3693,12 @@ bool h_changed_mid(const ems_gpu *h) {
 // Whether steps can run fused: not while an H source needs the serial gap
 // between the H and E updates (GAP_B, mod.rs:899-913; pool.rs:870-875).
 // The fused kernel keeps the slabs that reach a tile in a 32-bit mask.
-bool fused_eligible(const ems_gpu *h) {
+bool fusable(const ems_gpu *h) {
   size_t ns = 0;
   for (auto &s : h->slabs) ns += s.len != 0;
-  return h->fused && !has_hsrc(h) && !has_magnetic_poles(h) && !has_gap_kernels(h) &&
-         !has_upml(h) && ns <= 32;
+  return !has_hsrc(h) && !has_magnetic_poles(h) && !has_gap_kernels(h) && !has_upml(h) && ns <= 32;
 }
+bool fused_eligible(const ems_gpu *h) { return h->fused && fusable(h); }
 
 // Whether the quad kernels take this grid: a plane's byte offsets in 32
 // bits.
@@ -4821,7 +4822,7 @@ void advance_counts(ems_gpu *h, uint64_t steps) {
     o.count += (b + o.interval - 1) / o.interval - (a + o.interval - 1) / o.interval;
   }
   h->step += steps;
-  if (fused_eligible(h)) h->lock ^= (int)(steps & 1);
+  if (h->counts && fusable(h)) h->lock ^= (int)(steps & 1);
 }
 
 // Scratch of one evaluation, in doubles: a sum per H row (nx * (3 ny - 2)),
@@ -6110,7 +6111,7 @@ int ems_gpu_set_schedule(ems_gpu *h, int fused, int tile_rows, int x_chunks) {
   h->packed = fused == 4 || fused == 5;
   h->band = fused == 6;
   if (x_chunks < 0) return fail(h, EMS_E_INVALID, "x_chunks must be >= 0");
-  h->fused = fused != 0;
+  h->fused = h->counts = fused != 0;
   h->auto_sched = false;
   if (tile_rows) h->tj = tile_rows;
   h->nchunk = x_chunks;
@@ -6842,6 +6843,36 @@ void batch_drop_graphs(ems_gpu_batch *b) {
   b->active.clear();
 }
 
+// The schedule of a batch on its models while this lives, their own after.
+struct BatchSchedule {
+  struct Own {
+    ems_gpu *h;
+    bool auto_sched, fused, prefetch, rows, packed, band;
+    int tj, nchunk;
+  };
+  std::vector<Own> own;
+  BatchSchedule(const ems_gpu_batch *b, const std::vector<int> &act) {
+    for (int q : act) {
+      ems_gpu *h = b->m[q];
+      own.push_back({h, h->auto_sched, h->fused, h->prefetch, h->rows, h->packed, h->band, h->tj,
+                     h->nchunk});
+      h->auto_sched = false, h->fused = true, h->counts = true;
+      h->rows = false, h->band = false;
+      h->prefetch = b->prefetch, h->packed = b->packed, h->tj = b->tj, h->nchunk = b->nchunk;
+    }
+  }
+  ~BatchSchedule() {
+    for (const Own &o : own) {
+      ems_gpu *h = o.h;
+      h->auto_sched = o.auto_sched, h->fused = o.fused, h->prefetch = o.prefetch;
+      h->rows = o.rows, h->packed = o.packed, h->band = o.band, h->tj = o.tj;
+      h->nchunk = o.nchunk;
+    }
+  }
+  BatchSchedule(const BatchSchedule &) = delete;
+  BatchSchedule &operator=(const BatchSchedule &) = delete;
+};
+
 // Writes the per-model launch arguments of `act` for both parities.
 // Whether the batch steps with the quad kernels instead of the packed rows
 // (256 patch antennas, 30 M nodes of which the CPML holds 63 %: 1.13
@@ -7138,26 +7169,27 @@ int ems_gpu_batch_run(ems_gpu_batch *b, const uint8_t *active, uint64_t n) {
     if (!active || active[q]) act.push_back((int)q);
   if (act.empty() || n == 0) return EMS_OK;
   const int par = b->m[act[0]]->par, lock = b->m[act[0]]->lock;
-  std::vector<int> boffs;
   for (int q : act) {
     ems_gpu *h = b->m[q];
     if (h->dead) return bfail(b, EMS_E_DEVICE, "model " + std::to_string(q) + ": " + h->err);
-    if (h->auto_sched || !h->fused) drop_graphs(h);  // (captured for the unfused schedule)
-    h->auto_sched = false;
-    h->fused = true, h->rows = false, h->band = false, h->prefetch = b->prefetch, h->tj = b->tj;
-    h->packed = b->packed;
-    h->nchunk = b->nchunk;
     for (auto &o : h->ops)
       if (o.type == OP_MUR)
         return bfail(b, EMS_E_UNSUPPORTED,
                      "model " + std::to_string(q) + " has a Mur boundary (not batched)");
-    if (!use_fused(h))
+    if (!fusable(h))
       return bfail(b, EMS_E_UNSUPPORTED,
                    "model " + std::to_string(q) +
                        " needs the unfused schedule (H source, magnetic poles, plane wave, "
                        "cut-face currents, openEMS PML layers or more than 32 CPML slabs)");
     if (((h->step ^ b->m[act[0]]->step) & 1) && h->lock != lock)
       return bfail(b, EMS_E_INVALID, "models of a batch step in lockstep");
+  }
+  // The models run on the batch's schedule until this call ends, then have
+  // their own again.
+  BatchSchedule own(b, act);
+  std::vector<int> boffs;
+  for (int q : act) {
+    ems_gpu *h = b->m[q];
     h->boff = h->par ^ par;
     boffs.push_back(h->boff);
     const int rc = prepare(h, n, false);

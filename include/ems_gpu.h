@@ -378,11 +378,12 @@ int ems_gpu_merged_state(ems_gpu *h, int id, double *cur, double *circ);
  * models): engines stepped together, one fused launch over the tiles of
  * every active model and one launch for all their post-E gaps per step,
  * captured in graphs on the batch's own stream. Every model computes what
- * its own engine would, bit for bit. The models must all run the fused
- * schedule, with one curl order, and be in step with each other (same
- * step parity, of all steps or of those not taken on schedule 0); a handle
- * listed twice is refused. The batch holds the handles; it does not own
- * them. ems_run_until_batch with an odd check
+ * its own engine would, bit for bit. The models must all be able to run
+ * the fused schedule, with one curl order, and be in step with each other
+ * (same step parity, of all steps or of those not taken on schedule 0); a
+ * handle listed twice is refused. The batch holds the handles; it does not
+ * own them, and its runs leave each model the schedule that it has by itself
+ * (ems_gpu_set_schedule). ems_run_until_batch with an odd check
  * interval can stop models at checks an odd number of steps apart: a later
  * ems_gpu_batch_run over all of them is then refused with EMS_E_INVALID
  * ("models of a batch step in lockstep"); run such models in separate

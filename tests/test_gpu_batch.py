@@ -138,7 +138,7 @@ def test_batch_after_single_runs():
     batch = E.EngineBatch([a, b])
     for n in (2, 21):
         batch.run(n)
-    a.run(2)  # (on the schedule the batch left it on)
+    a.run(2)  # (on the schedule it had before)
     c.run(28)
     d.run(26)
     for x, y in ((a, c), (b, d)):
@@ -177,3 +177,44 @@ def test_batch_takes_models_of_equal_steps_on_any_schedule(packed):
     batch.close()
     for e in (a, b, c, d, x, y):
         e.close()
+
+
+def test_batch_leaves_the_models_their_schedules():
+    """After a batch's run, and after a run it refuses, every model steps on
+    its own schedule: the engine's choice (the unfused kernels), a fused
+    tiling or the unfused one that were set; the same bits as alone."""
+    ms = models()[:3]
+
+    def three():
+        es = [engine(m)[0] for m in ms]
+        es[1].set_schedule(2, 3, 2)
+        es[2].set_schedule(0)
+        return es
+
+    def own(es):  # (a fused step has no E kernel of its own)
+        return [e.traffic_model()[1] > 0.0 for e in es]
+    es, alone = three(), three()
+    assert own(es) == [True, False, True]
+    for packed in (False, True):
+        b = E.EngineBatch(es)
+        b.set_schedule(7, 2, packed=packed)
+        b.run(5)
+        assert own(es) == [True, False, True]
+        b.close()
+        for e in es:
+            e.run(3)
+    h_source, _ = engine(ms[0])
+    h_source.add_operator(E.EdgeSource(E.Waveform.gaussian(2e9, 1e9)).kind(E.SourceKind.SoftH)
+                          .edge(E.Axis.X, [6, 6, 3], 1.0))
+    b = E.EngineBatch(es + [h_source])
+    with pytest.raises(E.EmsError, match="unfused"):
+        b.run(2)
+    assert own(es) == [True, False, True]
+    b.close()
+    for e, f in zip(es, alone):
+        e.run(18)
+        f.run(34)
+        same_fields(e, f)
+        e.close()
+        f.close()
+    h_source.close()
