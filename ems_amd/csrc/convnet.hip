@@ -759,7 +759,6 @@ struct ems_cn {
   float sw = 0.0f;
   Buf didx;
   float *res = nullptr;             // pinned: loss, gradient norm
-  hipEvent_t done = nullptr;        // res written
   std::string err;
 };
 
@@ -1038,7 +1037,6 @@ int ems_cn_create(int cin, int cout, int channels, int layers, const int32_t *di
     n->lay.push_back(y);
   }
   if (hipStreamCreateWithFlags(&n->stream, hipStreamNonBlocking) != hipSuccess ||
-      hipEventCreateWithFlags(&n->done, hipEventDisableTiming) != hipSuccess ||
       hipMalloc(&n->p, n->np * 4) != hipSuccess || hipMalloc(&n->g, n->np * 4) != hipSuccess ||
       hipMalloc(&n->m, n->np * 4) != hipSuccess || hipMalloc(&n->v, n->np * 4) != hipSuccess ||
       hipMalloc(&n->w, n->nw * sizeof(u32x4)) != hipSuccess ||
@@ -1068,7 +1066,6 @@ void ems_cn_destroy(ems_cn *n) {
     for (auto &q : *v)
       if (q.d) (void)hipFree(q.d);
   if (n->res) (void)hipHostFree(n->res);
-  if (n->done) (void)hipEventDestroy(n->done);
   if (n->stream) (void)hipStreamDestroy(n->stream);
   delete n;
 }
@@ -1155,11 +1152,8 @@ int ems_cn_train_batch(ems_cn *n, const int32_t *idx, int B, int t0, float lr, f
                      n->np, lr, b1, b2, 1e-8f, c1, c2, clip, n->part.d, s.nb, n->spart.d, s.nsb,
                      s.inv, n->sq.d, s.nsq, n->res);
   CCK(n, hipGetLastError());
-  CCK(n, hipEventRecord(n->done, n->stream));
   n->w_ok = n->wr_ok = false;
-  // the next step's weights, while the host looks at the loss
-  if ((rc = weights_train(n))) return rc;
-  CCK(n, hipEventSynchronize(n->done));
+  CCK(n, hipStreamSynchronize(n->stream));
   if (loss) *loss = n->res[0];
   if (grad_norm) *grad_norm = n->res[1];
   return EMS_OK;
