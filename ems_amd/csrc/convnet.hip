@@ -803,6 +803,10 @@ int ensure_predict(ems_cn *n, int B, int T) {
 int ensure_train(ems_cn *n, int B, int T) {
   const size_t BT = (size_t)B * T;
   int rc;
+  // (with the first training call: a network that only predicts has neither)
+  if (!n->wr) CCK(n, hipMalloc(&n->wr, n->nr * sizeof(float)));
+  if (!n->res)
+    CCK(n, hipHostMalloc((void **)&n->res, 2 * sizeof(float), hipHostMallocDefault));
   n->h.resize(n->L), n->a.resize(n->L);
   if ((rc = grow(n, n->hx, BT * n->cin))) return rc;
   if ((rc = grow(n, n->hy, BT * n->cout))) return rc;
@@ -1040,11 +1044,9 @@ int ems_cn_create(int cin, int cout, int channels, int layers, const int32_t *di
       hipMalloc(&n->p, n->np * 4) != hipSuccess || hipMalloc(&n->g, n->np * 4) != hipSuccess ||
       hipMalloc(&n->m, n->np * 4) != hipSuccess || hipMalloc(&n->v, n->np * 4) != hipSuccess ||
       hipMalloc(&n->w, n->nw * sizeof(u32x4)) != hipSuccess ||
-      hipMalloc(&n->wr, n->nr * sizeof(float)) != hipSuccess ||
       hipMalloc(&n->dlay, n->lay.size() * sizeof(CnLayer)) != hipSuccess ||
-      hipHostMalloc((void **)&n->res, 2 * sizeof(float), hipHostMallocDefault) != hipSuccess ||
-      hipMemcpy(n->dlay, n->lay.data(), n->lay.size() * sizeof(CnLayer), hipMemcpyHostToDevice) !=
-          hipSuccess) {
+      hipMemcpyAsync(n->dlay, n->lay.data(), n->lay.size() * sizeof(CnLayer),
+                     hipMemcpyHostToDevice, n->stream) != hipSuccess) {
     ems_cn_destroy(n);
     return EMS_E_DEVICE;
   }

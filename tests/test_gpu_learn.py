@@ -5,9 +5,12 @@ the same parameters and inputs. The device accumulates in f32 in its own
 order (multiply-adds contracted), so values agree to a tolerance: 2e-5 of
 the largest magnitude for outputs, 2e-4 for gradients and 1e-5 for
 parameters after a step."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
+from ems_amd import _native as nat
 from oracle import convnet as O
 
 pytestmark = pytest.mark.gpu
@@ -206,3 +209,28 @@ def test_infinite_and_tiny_inputs():
     assert np.all(np.isfinite(got))
     _close(got, O.forward(s, p.astype(np.float64), x.astype(np.float64)), 2e-5)
     n.close()
+
+
+def test_prediction_needs_no_training_memory():
+    """Creating a network and predicting allocate the parameters, the
+    gradient, Adam's two moments and the packed bf16 weights (18 bytes a
+    parameter and the padded first and last layers); the rows that training
+    reads come with the first training call."""
+    cin, cout, ch, dil = 32, 32, 1024, (1, 2, 4)
+    x, y = np.zeros((1, cin, 16), np.float32), np.zeros((1, cout, 16), np.float32)
+
+    def free():  # (the runtime that the library is linked with)
+        a, b = C.c_size_t(), C.c_size_t()
+        assert nat.lib.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+        return a.value
+    small = _net(cin, cout, 64, (1, 2), 1)  # (the runtime's own first allocations)
+    small.loss_grad(x, y, 0)
+    start = free()
+    n = _net(cin, cout, ch, dil, 1)
+    n.forward(x)
+    used = start - free()
+    assert used < 20 * n.param_count, used / n.param_count
+    n.loss_grad(x, y, 0)
+    assert start - free() > used + 7 * n.param_count
+    n.close()
+    small.close()
