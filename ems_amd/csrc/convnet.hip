@@ -819,10 +819,12 @@ int ensure_train(ems_cn *n, int B, int T) {
   if ((rc = grow(n, n->gh, BT * n->C))) return rc;
   for (auto &d : n->dz)
     if ((rc = grow(n, d, BT * n->C))) return rc;
-  const size_t rs = ((size_t)B * n->cout + 7) / 8 * 8;
   if ((rc = grow(n, n->part, blocks(BT * n->cout)))) return rc;
-  if ((rc = grow(n, n->spart, (size_t)((T + 63) / 64) * (rs / 8)))) return rc;
-  if ((rc = grow(n, n->serr, rs * T))) return rc;
+  if (n->sw != 0.0f) {  // the spectral term's errors and partial sums
+    const size_t rs = ((size_t)B * n->cout + 7) / 8 * 8;
+    if ((rc = grow(n, n->spart, (size_t)((n->slen + 63) / 64) * (rs / 8)))) return rc;
+    if ((rc = grow(n, n->serr, rs * n->slen))) return rc;
+  }
   if ((rc = grow(n, n->sq, blocks(n->np)))) return rc;
   return grow(n, n->didx, B);
 }

@@ -211,6 +211,13 @@ def test_infinite_and_tiny_inputs():
     n.close()
 
 
+def _free():
+    """Free device memory (the runtime that the library is linked with)."""
+    a, b = C.c_size_t(), C.c_size_t()
+    assert nat.lib.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+    return a.value
+
+
 def test_prediction_needs_no_training_memory():
     """Creating a network and predicting allocate the parameters, the
     gradient, Adam's two moments and the packed bf16 weights (18 bytes a
@@ -218,19 +225,34 @@ def test_prediction_needs_no_training_memory():
     reads come with the first training call."""
     cin, cout, ch, dil = 32, 32, 1024, (1, 2, 4)
     x, y = np.zeros((1, cin, 16), np.float32), np.zeros((1, cout, 16), np.float32)
-
-    def free():  # (the runtime that the library is linked with)
-        a, b = C.c_size_t(), C.c_size_t()
-        assert nat.lib.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
-        return a.value
     small = _net(cin, cout, 64, (1, 2), 1)  # (the runtime's own first allocations)
     small.loss_grad(x, y, 0)
-    start = free()
+    start = _free()
     n = _net(cin, cout, ch, dil, 1)
     n.forward(x)
-    used = start - free()
+    used = start - _free()
     assert used < 20 * n.param_count, used / n.param_count
     n.loss_grad(x, y, 0)
-    assert start - free() > used + 7 * n.param_count
+    assert start - _free() > used + 7 * n.param_count
     n.close()
     small.close()
+
+
+def test_training_memory_of_one_long_trace():
+    """A batch of one trace takes nine buffers of its length (inputs, targets,
+    output, its gradient, the hidden layer's two, three of the backward pass);
+    the spectral term's errors, padded to eight rows, come with that term."""
+    T = 1 << 24
+    n = _net(1, 1, 1, (1, 2), 1)
+    x = np.zeros((1, 1, T), np.float32)
+    n.loss_grad(x[:, :, :64], x[:, :, :64], 0)
+    start = _free()
+    n.loss_grad(x, x, 0)
+    used = start - _free()
+    assert used < 9.5 * 4 * T, used / (4 * T)
+    n.set_spectral(np.eye(64, dtype=np.float32), 8, 0.5)
+    y = np.full((1, 1, T), 1.0, np.float32)
+    loss, _ = n.loss_grad(x, y, 0)
+    # (without biases zeros give zeros: d = -1, d^T K d = 64)
+    assert abs(loss - (1.0 + 0.5 * 64)) < 1e-4
+    n.close()
