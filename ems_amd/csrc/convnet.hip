@@ -271,15 +271,20 @@ constexpr int MW = 8;
 constexpr int AHEAD = 4;  // source channels loaded ahead
 __device__ __forceinline__ void cn_sums(const float *__restrict__ src, int ns,
                                         const float *__restrict__ w, int groups, int T, int dil,
-                                        int dir, int t, float acc[MW]) {
-  // per tap: the lane's sample (clamped) and whether it is one
+                                        int dir, unsigned t0, unsigned t, float acc[MW]) {
+  // per tap: the lane's sample (clamped) and whether it is one; byte offsets
+  // from the first sample that the wave may read, so that 32 bits hold them
+  // for sequences of any length (and dilations below 2^27)
+  const int64_t reach = (int64_t)t0 - (int64_t)dil * (CN_K - 1);
+  const int64_t first = dir > 0 ? (int64_t)t0 : (reach > 0 ? reach : 0);
+  src += first;
   unsigned at[CN_K];
   bool in[CN_K];
 #pragma unroll
   for (int k = 0; k < CN_K; k++) {
     const int64_t s = (int64_t)t + (int64_t)dir * dil * (CN_K - 1 - k);
     in[k] = s >= 0 && s < T;
-    at[k] = in[k] ? 4u * (unsigned)s : 0u;
+    at[k] = in[k] ? 4u * (unsigned)(s - first) : 0u;
   }
   float x[AHEAD][CN_K];
 #pragma unroll
@@ -326,25 +331,27 @@ struct FmaArgs {
   float *dz;             // gradient: dz of the layer below
   int last;              // forward: the last layer
 };
-__device__ __forceinline__ void cn_place(const FmaArgs &p, int &b, int &m0, int &t0) {
+__device__ __forceinline__ void cn_place(const FmaArgs &p, int &b, int &m0, unsigned &t0) {
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const unsigned id = blockIdx.x * 4u + wv;
   const unsigned g = id % (unsigned)p.groups, q = id / (unsigned)p.groups;
   b = (int)(q / (unsigned)p.tiles);
-  t0 = (int)(q - (unsigned)b * (unsigned)p.tiles) * 64;
+  t0 = (q - (unsigned)b * (unsigned)p.tiles) * 64;
   m0 = (int)g * MW;
 }
 
 __global__ void __launch_bounds__(256) cn_fwd(FmaArgs p, int B) {
-  int b, m0, t0;
+  int b, m0;
+  unsigned t0;
   cn_place(p, b, m0, t0);
   if (b >= B) return;
-  const int t = t0 + (int)(threadIdx.x & 63);
+  const unsigned t = t0 + (threadIdx.x & 63);
   float acc[MW];
 #pragma unroll
   for (int m = 0; m < MW; m++) acc[m] = m0 + m < p.mc ? cn_uniform(p.bias, m0 + m) : 0.0f;
-  cn_sums(p.src + (size_t)b * p.ns * p.T, p.ns, p.w + m0 * CN_K, p.groups, p.T, p.dil, -1, t, acc);
-  if (t >= p.T) return;
+  cn_sums(p.src + (size_t)b * p.ns * p.T, p.ns, p.w + m0 * CN_K, p.groups, p.T, p.dil, -1, t0, t,
+          acc);
+  if (t >= (unsigned)p.T) return;
 #pragma unroll
   for (int m = 0; m < MW; m++) {
     if (m0 + m >= p.mc) continue;
@@ -365,15 +372,17 @@ __global__ void __launch_bounds__(256) cn_fwd(FmaArgs p, int B) {
 // The gradient of a layer's input: gh = [gh +] sums, and dz = gh (1 - a^2)
 // of the layer below.
 __global__ void __launch_bounds__(256) cn_bwd(FmaArgs p, int B) {
-  int b, m0, t0;
+  int b, m0;
+  unsigned t0;
   cn_place(p, b, m0, t0);
   if (b >= B) return;
-  const int t = t0 + (int)(threadIdx.x & 63);
+  const unsigned t = t0 + (threadIdx.x & 63);
   float acc[MW];
 #pragma unroll
   for (int m = 0; m < MW; m++) acc[m] = 0.0f;
-  cn_sums(p.src + (size_t)b * p.ns * p.T, p.ns, p.w + m0 * CN_K, p.groups, p.T, p.dil, 1, t, acc);
-  if (t >= p.T) return;
+  cn_sums(p.src + (size_t)b * p.ns * p.T, p.ns, p.w + m0 * CN_K, p.groups, p.T, p.dil, 1, t0, t,
+          acc);
+  if (t >= (unsigned)p.T) return;
 #pragma unroll
   for (int m = 0; m < MW; m++) {
     if (m0 + m >= p.mc) continue;
@@ -402,20 +411,23 @@ __global__ void __launch_bounds__(256, 1) cn_wgrad(const float *__restrict__ dz,
   __shared__ float red[RB][256];
   const int tiles = (cin + CI - 1) / CI;
   const int co0 = (int)blockIdx.x / tiles * CO, ci0 = (int)blockIdx.x % tiles * CI;
-  const int n = B * T;
+  // this thread's samples: every 256th of the B T
+  const int n = (int)(((int64_t)B * T - (int)threadIdx.x + 255) / 256);
   float acc[NA];  // [co][ci][k], then the bias sums
 #pragma unroll
   for (int q = 0; q < NA; q++) acc[q] = 0.0f;
   int lags[CN_K];  // (from T on: no samples)
 #pragma unroll
   for (int k = 0; k < CN_K; k++) lags[k] = (int)min((int64_t)T, (int64_t)dil * (CN_K - 1 - k));
-  // A thread's samples, 256 apart: sample i of the B T has time t, and od and
-  // ox are the byte offsets of (sequence, channel 0, t) in dz and x.
+  // Sample i of them has time t, and od and ox are the byte offsets of
+  // (sequence, channel 0, t) in dz and x.
   // (Past the end the last is read again, channels past the last read the
   // last, and a lag past the start reads x at t: none of those is added.)
-  int i = threadIdx.x, t = i % T;
-  size_t od = 4 * ((size_t)(i / T) * con * T + t), ox = 4 * ((size_t)(i / T) * cin * T + t);
-  if (i >= n) od = ox = 0, t = 0;
+  int i = 0;
+  int t = (int)(threadIdx.x % T);
+  const size_t seq = threadIdx.x / T;
+  size_t od = 4 * (seq * con * T + t), ox = 4 * (seq * cin * T + t);
+  if (n == 0) od = ox = 0, t = 0;
   float d[D][CO], v[D][CI][CN_K];
   int ts[D];
   auto load = [&](int a) {
@@ -430,20 +442,21 @@ __global__ void __launch_bounds__(256, 1) cn_wgrad(const float *__restrict__ dz,
       for (int c = 0; c < CI; c++)
         v[a][c][k] = *(const float *)((const char *)(x + (size_t)min(ci0 + c, cin - 1) * T) + o);
     }
-    i += 256;
-    if (i < n) {
-      t += 256, od += 1024, ox += 1024;
-      while (t >= T) {  // into the next sequence
-        t -= T;
+    if (++i < n) {
+      od += 1024, ox += 1024;
+      unsigned next = (unsigned)t + 256;
+      while (next >= (unsigned)T) {  // into the next sequence
+        next -= T;
         od += 4 * (size_t)(con - 1) * T, ox += 4 * (size_t)(cin - 1) * T;
       }
+      t = (int)next;
     }
   };
 #pragma unroll
   for (int a = 0; a < D; a++) load(a);
-  for (int u = threadIdx.x; u < n;) {
+  for (int u = 0; u < n;) {
 #pragma unroll
-    for (int a = 0; a < D; a++, u += 256) {
+    for (int a = 0; a < D; a++, u++) {
       if (u < n) {
 #pragma unroll
         for (int e = 0; e < CI; e++)
@@ -906,7 +919,7 @@ int predict(ems_cn *n, int B, int T) {
 
 template <bool FWD>
 int launch_fma(ems_cn *n, FmaArgs a, int B) {
-  a.tiles = (a.T + 63) / 64;
+  a.tiles = (a.T - 1) / 64 + 1;
   a.groups = (a.mc + MW - 1) / MW;
   const dim3 g((unsigned)(((size_t)B * a.tiles * a.groups + 3) / 4)), t(256);
   if (FWD) hipLaunchKernelGGL(cn_fwd, g, t, 0, n->stream, a, B);

@@ -256,3 +256,28 @@ def test_training_memory_of_one_long_trace():
     # (without biases zeros give zeros: d = -1, d^T K d = 64)
     assert abs(loss - (1.0 + 0.5 * 64)) < 1e-4
     n.close()
+
+
+def test_sequences_past_2_to_the_30():
+    """A training step on two traces of more than 2^30 samples (2^31 in all)
+    whose last 4096 samples alone are not zero, the loss over the last 2048:
+    what a step on those 4096 gives. The sums of a weight's gradient hold the
+    same terms in other partial sums (1e-4 of the norm); a learning rate of
+    1e-3 moves every parameter by that much, the gradient's sign deciding."""
+    tail, T = 4096, (1 << 30) + 4096
+    rng = np.random.default_rng(3)
+    xs = rng.standard_normal((1, 1, tail)).astype(np.float32)
+    ys = rng.standard_normal((1, 1, tail)).astype(np.float32)
+    got = []
+    for length in (tail, T):
+        n = _net(1, 1, 1, (3, 5), 1)
+        x, y = np.zeros((1, 1, length), np.float32), np.zeros((1, 1, length), np.float32)
+        x[:, :, -tail:], y[:, :, -tail:] = xs, ys
+        n.set_data(x, y)
+        del x, y
+        loss = n.train_batch([0, 0], length - 2048, 1e-3)
+        got.append((loss, n.last_grad_norm, n.params()))
+        n.close()
+    (l0, g0, p0), (l1, g1, p1) = got
+    assert g0 > 0.0 and abs(l1 - l0) <= 1e-5 * l0 and abs(g1 - g0) <= 1e-4 * g0
+    assert np.abs(p1 - p0).max() <= 1e-5
