@@ -695,13 +695,17 @@ __global__ void __launch_bounds__(256) cn_finish(const float *part, int nb, cons
 
 // Adam on the f32 master parameters, the gradient scaled to the norm `clip`
 // where it is longer (every block adds up the norm's partial sums itself);
-// block 0 leaves the loss and the norm for the host.
+// block 0 leaves the loss and the norm for the host. A weight's new bf16
+// value goes to training's rows (cn_rows) at once: packing them afresh cost
+// the next step 4 us and a launch.
 __global__ void __launch_bounds__(256) cn_adam(float *__restrict__ p, const float *__restrict__ g,
                                                float *__restrict__ m, float *__restrict__ v,
                                                size_t n, float lr, float b1, float b2, float eps,
                                                float c1, float c2, float clip, const float *part,
                                                int nb, const float *spart, int nsb, float inv,
-                                               const float *sq, int nsq, float *res) {
+                                               const float *sq, int nsq, float *res,
+                                               const CnLayer *__restrict__ layers, int L,
+                                               float *__restrict__ rows) {
   __shared__ double red[256];
   const double n2 = cn_total(sq, nsq, red);
   const double gn = sqrt(n2);
@@ -714,7 +718,17 @@ __global__ void __launch_bounds__(256) cn_adam(float *__restrict__ p, const floa
   const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
   m[i] = mi;
   v[i] = vi;
-  p[i] = p[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+  const float pi = p[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+  p[i] = pi;
+  int l = L - 1;
+  while (l > 0 && layers[l].woff > i) l--;
+  const CnLayer y = layers[l];
+  const size_t w = i - y.woff;
+  if (w >= (size_t)y.co * y.ci * CN_K) return;  // a bias
+  const int k = (int)(w % CN_K), ci = (int)(w / CN_K % y.ci), co = (int)(w / CN_K / y.ci);
+  const float q = __uint_as_float((uint32_t)f32_to_bf16(pi) << 16);
+  rows[y.f + (((size_t)ci * y.gf + co / MW) * CN_K + k) * MW + co % MW] = q;
+  rows[y.b + (((size_t)co * y.gb + ci / MW) * CN_K + k) * MW + ci % MW] = q;
 }
 
 // Samples idx[] of a dataset [n][c][T] into a batch.
@@ -740,7 +754,8 @@ struct ems_cn {
   size_t np = 0;                    // parameters
   float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;
   // the weights' bf16 values as prediction (cn_pack) and training (cn_rows)
-  // read them, each made when first needed after a change, and their table
+  // read them, each made when first needed after a change (training's rows
+  // follow its steps), and their table
   std::vector<CnLayer> lay;
   CnLayer *dlay = nullptr;
   u32x4 *w = nullptr;
@@ -1167,9 +1182,9 @@ int ems_cn_train_batch(ems_cn *n, const int32_t *idx, int B, int t0, float lr, f
   const float c1 = 1.0f - std::pow(b1, (float)n->step), c2 = 1.0f - std::pow(b2, (float)n->step);
   hipLaunchKernelGGL(cn_adam, dim3(blocks(n->np)), dim3(256), 0, n->stream, n->p, n->g, n->m, n->v,
                      n->np, lr, b1, b2, 1e-8f, c1, c2, clip, n->part.d, s.nb, n->spart.d, s.nsb,
-                     s.inv, n->sq.d, s.nsq, n->res);
+                     s.inv, n->sq.d, s.nsq, n->res, n->dlay, n->L, n->wr);
   CCK(n, hipGetLastError());
-  n->w_ok = n->wr_ok = false;
+  n->w_ok = false;
   CCK(n, hipStreamSynchronize(n->stream));
   if (loss) *loss = n->res[0];
   if (grad_norm) *grad_norm = n->res[1];

@@ -281,3 +281,22 @@ def test_sequences_past_2_to_the_30():
     (l0, g0, p0), (l1, g1, p1) = got
     assert g0 > 0.0 and abs(l1 - l0) <= 1e-5 * l0 and abs(g1 - g0) <= 1e-4 * g0
     assert np.abs(p1 - p0).max() <= 1e-5
+
+
+@pytest.mark.parametrize("shape", EDGES[:4], ids=str)
+def test_weight_rows_follow_the_optimizer(shape):
+    """Gradients after optimizer steps, whose weight rows the steps wrote, are
+    those of the same parameters packed afresh, bit for bit."""
+    cin, cout, ch, dil, B, T = shape
+    n, fresh = _net(cin, cout, ch, dil, 5), _net(cin, cout, ch, dil, 6)
+    rng = np.random.default_rng(T)
+    x = rng.standard_normal((B, cin, T)).astype(np.float32)
+    y = rng.standard_normal((B, cout, T)).astype(np.float32)
+    n.set_data(x, y)
+    for _ in range(3):
+        n.train_batch(np.arange(B), T // 3, 1e-2)
+        fresh.set_params(n.params())
+        for a, b in zip(n.loss_grad(x, y, 0), fresh.loss_grad(x, y, 0)):
+            assert np.array_equal(np.float32(a).view(np.uint32), np.float32(b).view(np.uint32))
+    n.close()
+    fresh.close()
