@@ -112,6 +112,7 @@ struct ConvArgs {
   int T, dil;
   int ml;      // samples per phase of a block
   int pt, nt;  // blocks along the phases and along a phase
+  unsigned blk0;  // the launch's first block
   const float *bias;
   const float *h_in;  // HIDDEN: the residual input, or null
   float *h_out;       // HIDDEN
@@ -136,7 +137,8 @@ __global__ void __launch_bounds__(512) cn_conv(ConvArgs p) {
   constexpr int LD = KC + 8;
   const int rows = cn_rows(p.ml), pr = p.ml + CN_K - 1;  // pr: rows of a phase
   const int tiles = p.pt * p.nt, mt0 = 2 * blockIdx.y;
-  const int b = blockIdx.x / tiles, tile = blockIdx.x - b * tiles;
+  const unsigned blk = p.blk0 + blockIdx.x;
+  const int b = (int)(blk / (unsigned)tiles), tile = (int)(blk - (unsigned)b * (unsigned)tiles);
   const int ph0 = tile / p.nt * (CN_TT / p.ml), m0 = tile % p.nt * p.ml;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nt = wv & 1, kh = wv >> 1;
   const bool two = mt0 + 1 < p.mt;
@@ -858,16 +860,21 @@ int ensure_train(ems_cn *n, int B, int T) {
 }
 
 template <int MODE, int KC>
-int launch_conv_k(ems_cn *n, const ConvArgs &a, int B) {
+int launch_conv_k(ems_cn *n, ConvArgs a, int B) {
   const size_t lds = cn_lds(a.ml, KC);
   if (lds > 64 * 1024)
     CCK(n, hipFuncSetAttribute((const void *)cn_conv<MODE, KC>,
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  hipLaunchKernelGGL((cn_conv<MODE, KC>),
-                     dim3((unsigned)a.pt * (unsigned)a.nt * (unsigned)B,
-                          (unsigned)((a.mt + 1) / 2)),
-                     dim3(512), lds, n->stream, a);
-  CCK(n, hipGetLastError());
+  // (a launch holds fewer than 2^32 threads)
+  constexpr uint64_t MOST = 1u << 22;
+  const uint64_t nb = (uint64_t)a.pt * a.nt * B;
+  for (uint64_t b0 = 0; b0 < nb; b0 += MOST) {
+    a.blk0 = (unsigned)b0;
+    hipLaunchKernelGGL((cn_conv<MODE, KC>),
+                       dim3((unsigned)std::min(MOST, nb - b0), (unsigned)((a.mt + 1) / 2)),
+                       dim3(512), lds, n->stream, a);
+    CCK(n, hipGetLastError());
+  }
   return 0;
 }
 

@@ -300,3 +300,16 @@ def test_weight_rows_follow_the_optimizer(shape):
             assert np.array_equal(np.float32(a).view(np.uint32), np.float32(b).view(np.uint32))
     n.close()
     fresh.close()
+
+
+def test_predictions_past_one_launch():
+    """More sequences than the blocks of one launch hold: every one's output
+    is that of its own short call."""
+    B = 9_000_000
+    n = _net(1, 1, 1, (1, 2), 4)
+    x = np.random.default_rng(1).standard_normal((B, 1, 1)).astype(np.float32)
+    got = n.forward(x)
+    for at in (0, (1 << 22) - 3, (1 << 23) - 3, B - 6):
+        few = n.forward(x[at:at + 6])
+        assert np.array_equal(got[at:at + 6].view(np.uint32), few.view(np.uint32)), at
+    n.close()
