@@ -6749,7 +6749,7 @@ int ems_gpu_traffic_model(ems_gpu *h, double out[3]) {
   double cp = 0;
   const bool fold[2] = {cpml_folded(h, 0), cpml_folded(h, 1)};
   for (auto &s : h->slabs) {
-    if (!use_fused(h) && fold[s.arg.e_side ? 1 : 0] && !s.out)
+    if (!use_fused(h) && fold[s.arg.e_side ? 1 : 0])
       out[s.arg.e_side ? 1 : 0] += 8.0 * (double)s.len;
     else
       cp += 28.0 * (double)s.len;

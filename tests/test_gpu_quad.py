@@ -99,3 +99,17 @@ def test_switches_agree(which):
     o.run(15)
     same_fields(g, o)
     assert np.array_equal(bits(pg.values()), bits(o.probe_values(po)))
+
+
+def test_traffic_model_of_a_step():
+    """The bytes of an unfused step do not depend on what ran before it."""
+    cells, layers = (13, 12, 19), [(f, 3) for f in ALL]
+    a, _ = build("gpu", cells, layers, 0, True, False)
+    b, _ = build("gpu", cells, layers, 0, True, False)
+    b.set_cpml_split(True)
+    b.set_schedule(1, 7, 0)
+    b.run(1)
+    b.set_schedule(0)
+    assert a.traffic_model() == b.traffic_model()
+    a.close()
+    b.close()
