@@ -3555,6 +3555,7 @@ struct ems_gpu {
   int lock = 0;    // parity of the steps but those taken on schedule 0 (batches)
   bool counts = true;  // whether its own steps count: not once set to 0, until a batch run
   int boff = 0;    // during a batch run: par relative to the batch's
+  uint64_t launch_gen = 0;  // counts what changed a step's launches (drop_graphs)
   Lane lanes[12]{};
   uint64_t lane_rows[12] = {0};
   std::vector<void *> lane_mem;
@@ -4548,6 +4549,7 @@ int enqueue_step(ems_gpu *h, int &par) {
 }
 
 void drop_graphs(ems_gpu *h) {
+  h->launch_gen++;
   for (int p = 0; p < 2; p++) {
     if (h->g1[p]) (void)hipGraphExecDestroy(h->g1[p]);
     if (h->gK[p]) (void)hipGraphExecDestroy(h->gK[p]);
@@ -6803,6 +6805,7 @@ struct ems_gpu_batch {
   bool prefetch = true, packed = false;
   std::vector<int> active;        // the set the graphs were captured for
   std::vector<int> boffs;         // their buffer parities relative to the first one
+  std::vector<uint64_t> gens;     // their launch_gen
   FusedArgs *d_args[2] = {nullptr, nullptr};
   GapArgs *d_gap[2] = {nullptr, nullptr};
   uint32_t *d_seg = nullptr;
@@ -7188,12 +7191,14 @@ int ems_gpu_batch_run(ems_gpu_batch *b, const uint8_t *active, uint64_t n) {
   // their own again.
   BatchSchedule own(b, act);
   std::vector<int> boffs;
+  std::vector<uint64_t> gens;
   for (int q : act) {
     ems_gpu *h = b->m[q];
     h->boff = h->par ^ par;
     boffs.push_back(h->boff);
     const int rc = prepare(h, n, false);
     if (rc) return bfail(b, rc, h->err);
+    gens.push_back(h->launch_gen);
     if (h->croff_wide)
       return bfail(b, EMS_E_UNSUPPORTED,
                    "model " + std::to_string(q) + " has a coefficient pool of 4 GiB or more");
@@ -7202,9 +7207,10 @@ int ems_gpu_batch_run(ems_gpu_batch *b, const uint8_t *active, uint64_t n) {
   const bool quads = batch_quads(b, act);
   if (quads)  // in place: the models' buffers do not change over the run
     for (size_t q = 0; q < act.size(); q++) boffs[q] = 2 + b->m[act[q]]->par;
-  // (graphs hold the models' buffers)
-  if (boffs != b->boffs || quads != b->quads) batch_drop_graphs(b);
+  // (graphs hold the models' buffers, and the launches of their poles)
+  if (boffs != b->boffs || quads != b->quads || gens != b->gens) batch_drop_graphs(b);
   b->boffs = boffs;
+  b->gens = gens;
   b->quads = quads;
   int rc = batch_args(b, act);
   if (rc) return rc;

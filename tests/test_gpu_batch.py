@@ -6,6 +6,7 @@ import pytest
 
 import ems_amd as E
 from ems_amd import workloads as W
+from ems_amd.dispersive import Dispersive, Field, Pole
 
 from test_gpu_parity import bits, same_fields
 
@@ -218,3 +219,41 @@ def test_batch_leaves_the_models_their_schedules():
         e.close()
         f.close()
     h_source.close()
+
+
+def poles(e):
+    """Lorentz poles in a block of a patch model's substrate."""
+    d = Dispersive.new()
+    w = 2.0 * np.pi * 4e9
+    d.fill_cells(e.grid, [(10, 18), (9, 20), (1, 6)], Field.Electric, [Pole.lorentz(w, w, 1e9)])
+    return e.add_operator(d)
+
+
+@pytest.mark.parametrize("graphs", [True, False])
+@pytest.mark.parametrize("packed", [False, True])
+def test_batch_with_poles(packed, graphs):
+    """A dispersive medium in one model of a batch, and one that another gets
+    between two runs (a step has other launches then)."""
+    ms = models()[:3]
+    single, batch = [engine(m) for m in ms], [engine(m) for m in ms]
+    b = E.EngineBatch([e for e, _ in batch])
+    b.set_schedule(7, 2, packed=packed)
+    b.set_graphs(graphs)
+    media = [(poles(es[1][0])) for es in (single, batch)]
+    late = []
+    for n in (37, 24, 1, 16):
+        b.run(n)
+        for e, _ in single:
+            e.run(n)
+        if not late:
+            late = [poles(es[2][0]) for es in (single, batch)]
+    for (e, p), (f, q) in zip(single, batch):
+        assert np.array_equal(bits(p.voltage()), bits(q.voltage()))
+        same_fields(e, f)
+    for x, y in (media, late):
+        for s, t in zip(x.state(Field.Electric), y.state(Field.Electric)):
+            assert np.array_equal(bits(np.asarray(s)), bits(np.asarray(t)))
+            assert np.abs(np.asarray(s)).max() > 0.0
+    b.close()
+    for e, _ in single + batch:
+        e.close()
