@@ -1115,7 +1115,7 @@ class Engine:
         the same values either way."""
         self._check(nat.ems_gpu_set_tile_classes(self._h, 1 if on else 0))
 
-    def set_unfused_prefetch(self, which: int = 11) -> None:
+    def set_unfused_prefetch(self, which: int = 15) -> None:
         """The unfused kernels: bits 0 (H) and 1 (E) take four nodes of a z
         row per thread (else one node, two x-planes); bits 2 (H) and 3 (E),
         with the side's bit 0 or 1, correct the side's CPML slabs inside the
