@@ -30,11 +30,17 @@ def graded(length: float, cells: int, alpha: float):
             for q in range(cells + 1)]
 
 
-# Schedule of the device engines the tests build: (fused, tile_rows, x_chunks)
-# and whether the tiled step corrects its z-normal CPML slabs outside itself,
-# splits its tiles in classes, and which unfused kernels load ahead.
+# Schedule of the device engines the tests build: (fused, tile_rows, x_chunks),
+# fused None leaving an engine as it is built, and whether the tiled step
+# corrects its z-normal CPML slabs outside itself, splits its tiles in
+# classes, and which unfused kernels run.
 SCHEDULE = {"fused": 1, "tile_rows": 0, "x_chunks": 0, "split": 0, "classes": 0,
-            "unfused_pf": 11}
+            "unfused_pf": 15}
+OWN = (None, 0, 0)
+
+
+def schedule_id(s):
+    return "own" if s[0] is None else "mode%d_tj%d_xc%d" % s[:3]
 
 
 def make(kind: str, grid, mats=None, faces=None, ts=None, threads=1, curl_order=0, pool=True):
@@ -44,10 +50,12 @@ def make(kind: str, grid, mats=None, faces=None, ts=None, threads=1, curl_order=
     lanes = E.coefficients(grid, mats, faces, dt)
     if kind == "gpu":
         e = E.Engine(grid, dt, lanes, curl_order=curl_order, pool=pool)
+        if SCHEDULE["fused"] is None:
+            return e
         e.set_schedule(SCHEDULE["fused"], SCHEDULE["tile_rows"], SCHEDULE["x_chunks"])
         e.set_cpml_split(bool(SCHEDULE.get("split", 0)))
         e.set_tile_classes(bool(SCHEDULE.get("classes", 0)))
-        e.set_unfused_prefetch(SCHEDULE.get("unfused_pf", 11))
+        e.set_unfused_prefetch(SCHEDULE.get("unfused_pf", 15))
         return e
     from oracle.bridge import OracleEngine
     return OracleEngine(grid, dt, lanes, curl_order=curl_order, threads=threads, pool=pool)

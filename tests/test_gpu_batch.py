@@ -9,6 +9,7 @@ from ems_amd import workloads as W
 from ems_amd.dispersive import Dispersive, Field, Pole
 
 from test_gpu_parity import bits, same_fields
+from test_gpu_quad import build as quad_build
 
 pytestmark = pytest.mark.gpu
 
@@ -127,7 +128,8 @@ def test_batch_refuses_models_out_of_step_and_duplicates():
     b.close()
 
 
-def test_batch_after_single_runs():
+@pytest.mark.parametrize("packed", [False, True])
+def test_batch_after_single_runs(packed):
     """Models that stepped on their own first, one of them on another
     schedule (the same steps taken, the state in another buffer), step on
     together like engines of their own."""
@@ -137,6 +139,7 @@ def test_batch_after_single_runs():
     a.run(3)
     b.run(3)
     batch = E.EngineBatch([a, b])
+    batch.set_schedule(7, 2, packed=packed)
     for n in (2, 21):
         batch.run(n)
     a.run(2)  # (on the schedule it had before)
@@ -254,6 +257,39 @@ def test_batch_with_poles(packed, graphs):
         for s, t in zip(x.state(Field.Electric), y.state(Field.Electric)):
             assert np.array_equal(bits(np.asarray(s)), bits(np.asarray(t)))
             assert np.abs(np.asarray(s)).max() > 0.0
+    b.close()
+    for e, _ in single + batch:
+        e.close()
+
+
+# Slabs that the quad kernels leave to others: z registered before y before
+# x, and two ends of z that meet in one quad. A batch of short rows with one
+# such model steps with the packed fused kernel.
+IRREGULAR = [((10, 11, 7), [(E.Face.ZMax, 3), (E.Face.YMin, 3), (E.Face.XMin, 4)]),
+             ((10, 10, 8), [(E.Face.ZMin, 3), (E.Face.ZMax, 4)])]
+REGULAR = ((13, 12, 19), [(f, 3) for f in E.Face])
+
+
+@pytest.mark.parametrize("prefetch", [False, True], ids=["noprefetch", "prefetch"])
+@pytest.mark.parametrize("curl", (0, 1))
+@pytest.mark.parametrize("irregular", IRREGULAR, ids=["z_first", "one_quad"])
+def test_batch_of_irregular_slabs(irregular, curl, prefetch):
+    """The packed fused kernel's batch (the irregular model), and the quad
+    kernels' between its runs (the others alone): models of both kinds as
+    alone, with and without chunks of x."""
+    shapes = [REGULAR, irregular, REGULAR]
+    single = [quad_build("gpu", c, l, curl, True, False) for c, l in shapes]
+    batch = [quad_build("gpu", c, l, curl, True, False) for c, l in shapes]
+    b = E.EngineBatch([e for e, _ in batch])
+    for chunks, n, act in ((0, 37, None), (3, 5, None), (3, 4, [True, False, True]), (3, 18, None)):
+        b.set_schedule(7, chunks, prefetch=prefetch, packed=True)
+        b.run(n, act)
+        for q, (e, _) in enumerate(single):
+            if act is None or act[q]:
+                e.run(n)
+    for (e, p), (f, r) in zip(single, batch):
+        same_fields(e, f)
+        assert np.array_equal(bits(p.values()), bits(r.values()))
     b.close()
     for e, _ in single + batch:
         e.close()

@@ -16,10 +16,10 @@ from test_gpu_parity import bits, same_fields
 
 pytestmark = pytest.mark.gpu
 
-SCHEDULES = [(0, 0, 0), (1, 7, 0), (1, 3, 4), (3, 7, 0)]
+SCHEDULES = [K.OWN, (0, 0, 0), (1, 7, 0), (1, 3, 4), (3, 7, 0)]
 
 
-@pytest.fixture(autouse=True, params=SCHEDULES, ids=lambda s: "mode%d_tj%d_xc%d" % s)
+@pytest.fixture(autouse=True, params=SCHEDULES, ids=K.schedule_id)
 def schedule(request):
     f, t, c = request.param
     old = dict(K.SCHEDULE)

@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 import ems_amd as E
+from cases import OWN, schedule_id
 from oracle.bridge import OracleEngine
 
 from test_gpu_parity import bits, same_fields
@@ -17,7 +18,7 @@ pytestmark = pytest.mark.gpu
 
 C0 = 299792458.0
 TAU = 2.8e-11
-SCHEDULES = [(0, 0, 0), (1, 7, 0), (2, 3, 2), (3, 7, 0), (4, 7, 0), (6, 8, 0)]
+SCHEDULES = [OWN, (0, 0, 0), (1, 7, 0), (2, 3, 2), (3, 7, 0), (4, 7, 0), (6, 8, 0)]
 
 
 def dgaussian(tau):
@@ -36,7 +37,8 @@ def build(kind, sched, openems=False, hold=0):
     lanes = E.coefficients(g, None, [E.FaceCondition.Pec] * 6, dt)
     if kind == "gpu":
         e = E.Engine(g, dt, lanes)
-        e.set_schedule(*sched)
+        if sched != OWN:
+            e.set_schedule(*sched)
     else:
         e = OracleEngine(g, dt, lanes, threads=2)
     m = E.MurBoundary.with_faces(e, [(f, C0 if f < 4 else 0.8 * C0) for f in E.Face])
@@ -52,7 +54,7 @@ def build(kind, sched, openems=False, hold=0):
     return e, p, q
 
 
-@pytest.mark.parametrize("sched", SCHEDULES, ids=lambda s: "mode%d_tj%d_xc%d" % s)
+@pytest.mark.parametrize("sched", SCHEDULES, ids=schedule_id)
 @pytest.mark.parametrize("variant", ["ems", "openems_hold"])
 def test_mur_box_matches_oracle(sched, variant):
     kw = {} if variant == "ems" else {"openems": True, "hold": 37}

@@ -6,11 +6,12 @@ import numpy as np
 import pytest
 
 import ems_amd as E
+from cases import OWN, schedule_id
 import openems_case as OC
 
 pytestmark = pytest.mark.gpu
 
-SCHEDULES = [(0, 0, 0), (1, 3, 0), (2, 7, 4), (3, 7, 0), (4, 7, 0), (5, 7, 2), (6, 4, 2), (6, 8, 0)]
+SCHEDULES = [OWN, (0, 0, 0), (1, 3, 0), (2, 7, 4), (3, 7, 0), (4, 7, 0), (5, 7, 2), (6, 4, 2), (6, 8, 0)]
 
 
 def bits(a):
@@ -28,12 +29,13 @@ def oracle_run():
     return o, {k: [o.probe_values(p) for p in ps] for k, ps in probes.items()}
 
 
-@pytest.mark.parametrize("sched", SCHEDULES, ids=lambda s: "mode%d_tj%d_xc%d" % s)
+@pytest.mark.parametrize("sched", SCHEDULES, ids=schedule_id)
 def test_gauss_soft_e_device(oracle_run, sched):
     o, want = oracle_run
     g, dt = OC.grid(), OC.dt()
     e = E.Engine(g, dt, OC.lanes(g, dt), curl_order=1)
-    e.set_schedule(*sched)
+    if sched != OWN:
+        e.set_schedule(*sched)
     probes = OC.build(e, g)
     e.run(OC.STEPS)
     for name, ps in probes.items():

@@ -15,7 +15,7 @@ from test_gpu_parity import bits, same_fields
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(autouse=True, params=[(0, 0, 0), (1, 7, 0)], ids=lambda s: "mode%d_tj%d_xc%d" % s)
+@pytest.fixture(autouse=True, params=[K.OWN, (0, 0, 0), (1, 7, 0)], ids=K.schedule_id)
 def schedule(request):
     f, t, c = request.param
     old = dict(K.SCHEDULE)
