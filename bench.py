@@ -201,8 +201,9 @@ def sweep(args, log) -> int:
             "traffic_measured_at": traffic_cfg,
             "bytes_per_launch": byt, "launch_ms": round(per_step * 1e3, 4),
             "models": int(sum(act)),
-            "timing": "wall clock of synchronised batch runs (64 steps, step and gap kernels); "
-                      "counters from a run without graphs"}
+            "timing": "a step (H, E and gap launches) by the wall clock of synchronised batch "
+                      "runs (64 steps); bytes and traffic of its H and E launches, counters "
+                      "from a run without graphs"}
     log(f"batched kernel: {per_step*1e3:.3f} ms per step over {sum(act)} models, "
         f"{achieved:.0f} GB/s algorithmic")
     d, same_steps = None, None
@@ -222,8 +223,8 @@ def sweep(args, log) -> int:
         "dtype": "f32", "data": "synthetic (seeded patch antennas)",
         "config": {"workload": f"patch_sweep_{n}", "models": n, "seed": args.seed,
                    "frequencies": 201, "end": "-40 dB energy decay",
-                   "schedule": {"kernel": "packed rows" if packed else f"tiled, {tj} rows",
-                                "x_chunks": args.x_chunks}},
+                   "schedule": ({"kernel": "unfused, four nodes per thread"} if packed else
+                                {"kernel": f"tiled, {tj} rows", "x_chunks": args.x_chunks})},
         "sequential_solves_per_hr": round(n / t_seq * 3600.0, 1) if t_seq else None,
         "speedup_vs_sequential": round(t_seq / t_bat, 3) if t_seq else None,
         "max_abs_dS11": d, "same_step_counts": same_steps,

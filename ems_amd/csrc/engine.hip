@@ -912,7 +912,11 @@ __global__ void __launch_bounds__(256, QW)
 }
 
 // The same over the models of a batch: what the kernels above take by
-// value, per model, and for each block its model.
+// value, per model, and for each block its model. The blocks always go in
+// runs of QUAD_RUN: contiguous eighths (quad_geom's order for one cached
+// grid) cut a batch's small models nowhere better and measured slower, 52.2
+// against 48.6 us a step for 8 patch antennas, 122.5 against 118.8 for 32,
+// 1102 against 1056 for 256.
 struct QuadModel {
   Fields f;
   Lanes L;
@@ -2487,10 +2491,12 @@ __device__ __forceinline__ bool mf_in_range(double s) {
 // k backward). Rows past the end solve 0 = 0. Returns false (x not written)
 // where a value leaves mf_div's range or is not finite.
 //
-// Bound by the chain of one row after the other: a product, a subtraction
-// and the quotient's five dependent operations per row and direction (some
-// 330 rows: 77 us; with an IEEE division, the row's length tested and one
-// row loaded ahead 97, and the large blocks' launch before it).
+// Bound by what the one lane issues per row and direction, 92 ns (300 to 900
+// rows): the seven operations that depend on the row before (a product, a
+// subtraction, the quotient's five) are a third of it at 5 ns each, the
+// range tests 7 ns (85 without them), the rest the operands' LDS loads, copies
+// and stores. Some 330 rows: 77 us; with an IEEE division, the row's length
+// tested and one row loaded ahead 97, and the large blocks' launch before it.
 __device__ __forceinline__ bool mf_narrow(const DevMerged &m, uint32_t r0, uint32_t nr,
                                           double *xs, uint32_t lane) {
   const uint32_t n4 = (nr + 3) / 4 * 4;
@@ -3707,11 +3713,13 @@ bool quad_ok(const ems_gpu *h) { return h->plane < ((size_t)1 << 29); }
 
 // An engine whose schedule nobody set steps unfused: the quad kernels read
 // and write each node twice a step instead of once, but at the copy rate,
-// without halo rows or a march along x, and with the CPML inside: 13.7
-// against 47 us per step on 25^3 nodes (the fused default, one block
-// marching 25 planes), 41 against 74 (132 x 98 x 75 nodes with CPML, the
-// best fused tiling), 2.60 against 2.83 ms (513^3, the best fused tiling;
-// the fused default 4.3).
+// without halo rows or a march along x, and with the CPML inside: 12.2
+// against 45 us per step on 25^3 nodes (the fused default, one block
+// marching 25 planes; 10.6 in 32 chunks), 33 against 75 (132 x 98 x 75
+// nodes with CPML, the best fused tiling), 2.60 against 2.83 ms (513^3, the
+// best fused tiling; the fused default 4.3). Slabs that quad_cpml_args leaves
+// to launches of their own take it back: 105 against 75 us (the same grid,
+// z registered first; the fused default 130), which the autotuner finds.
 bool use_fused(const ems_gpu *h) {
   return !(h->auto_sched && quad_ok(h)) && fused_eligible(h);
 }
@@ -4570,8 +4578,6 @@ int capture(ems_gpu *h, int steps, int par, hipGraphExec_t *out) {
   return 0;
 }
 
-// Uploads the operator and slab tables, and grows probe buffers to hold
-// `steps` more steps of samples.
 // Moves every lane's rows into one pool (a zero row first) and builds the
 // per-row offset table the fused kernel reads; the lanes then point into
 // the pool, so each coefficient is stored once.
@@ -4707,6 +4713,8 @@ int build_tile_classes(ems_gpu *h) {
   return 0;
 }
 
+// Uploads the operator and slab tables, and grows probe buffers to hold
+// `steps` more steps of samples.
 int prepare(ems_gpu *h, uint64_t steps, bool allow_split = true) {
   if (h->lanes_dirty) {
     drop_graphs(h);
@@ -6876,7 +6884,6 @@ struct BatchSchedule {
   BatchSchedule &operator=(const BatchSchedule &) = delete;
 };
 
-// Writes the per-model launch arguments of `act` for both parities.
 // Whether the batch steps with the quad kernels instead of the packed rows
 // (256 patch antennas, 30 M nodes of which the CPML holds 63 %: 1.13
 // against 1.24 ms a step; 8 antennas 50 against 74 us): every model's slabs
@@ -6944,6 +6951,8 @@ int batch_quad_args(ems_gpu_batch *b, const std::vector<int> &act) {
   return 0;
 }
 
+// Writes the per-model launch arguments of `act` (fused steps: for both
+// parities).
 int batch_args(ems_gpu_batch *b, const std::vector<int> &act) {
   if (b->quads) return batch_quad_args(b, act);
   const size_t n = act.size();
@@ -7001,8 +7010,6 @@ void batch_launch_tj(ems_gpu_batch *b, int par, int nm) {
                      2);
 }
 
-// One batched step from parity `par` (every active model holds its state
-// in fbuf[par]).
 // The models' dispersive media on the batch's stream (launch_poles).
 int batch_poles(ems_gpu_batch *b, const std::vector<int> &act, int stage, int par) {
   for (int q : act) {
@@ -7045,6 +7052,7 @@ int batch_enqueue_quads(ems_gpu_batch *b, const std::vector<int> &act) {
   return 0;
 }
 
+// One batched step from parity `par` (the first active model's; fused steps).
 int batch_enqueue_step(ems_gpu_batch *b, const std::vector<int> &act, int par) {
   if (b->quads) return batch_enqueue_quads(b, act);
   const int nm = (int)act.size();

@@ -1199,9 +1199,10 @@ def energy_many(engines: Sequence["Engine"], active: Optional[Sequence[bool]] = 
 
 
 class EngineBatch:
-    """Engines stepped together (include/ems_gpu.h batches): one fused launch
-    over the tiles of every active model per step, each model bit-identical
-    to stepping it alone. No reference counterpart (the reference runs one
+    """Engines stepped together (include/ems_gpu.h batches): one launch (short
+    rows: one per half-step) over every active model per step, each model
+    bit-identical to stepping it alone; a model's own schedule is for the
+    steps it takes by itself. No reference counterpart (the reference runs one
     model per engine); the run loop per model is run::drive
     (src/engine/run.rs:424-540)."""
 
@@ -1233,11 +1234,14 @@ class EngineBatch:
 
     def set_schedule(self, tile_rows: int = 7, x_chunks: int = 0, prefetch: bool = False,
                      packed: bool = False) -> None:
-        """The fused kernel of every model: tiled (tile height 3, 7 or 15) or
-        packed short rows (64 // nz whole rows per wave, every nz <= 64);
-        x chunks per model (0 automatic); the next-plane prefetch (off by
-        default: without it the kernels run eight waves per SIMD, and the
-        256-model patch batch steps in 1.201 ms against 1.336 with it)."""
+        """The kernels of every model: tiled fused (tile height 3, 7 or 15) or,
+        with `packed`, short rows (every nz <= 64): the unfused kernels of
+        four nodes per thread, or, where a model's CPML slabs are not in their
+        form, packed fused rows (64 // nz whole rows per wave). x chunks per
+        model (0 automatic) and the next-plane prefetch are the fused
+        kernels' (off by default: without it they run eight waves per SIMD;
+        the 256-model patch batch 1.201 ms a step against 1.336 with it, and
+        1.06 with the unfused kernels)."""
         mode = (4 if prefetch else 5) if packed else (1 if prefetch else 2)
         self._check(nat.ems_gpu_batch_set_schedule(self._h, mode, int(tile_rows), int(x_chunks)))
 

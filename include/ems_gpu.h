@@ -465,8 +465,11 @@ double ems_gpu_dt(const ems_gpu *h);
  * 4 packed short rows: 64 / nz whole k-rows per wave, nz <= 64, else the
  * tiled kernel; 5 the same without the prefetch); tile_rows 3, 7 or 15
  * (0 keeps the current); x_chunks 0 = automatic. Until this is called the
- * engine steps unfused (measured fastest at every size). Steps that need the serial gap between the H and
- * E updates (H sources) always run unfused. */
+ * engine steps unfused, which measured faster than the fused default at
+ * every size (a fused tiling of many x chunks can be as fast on the smallest
+ * boxes, and is faster where CPML slabs are not in the unfused kernels'
+ * form). Steps that need the serial gap between the H and E updates (H
+ * sources) always run unfused. */
 int ems_gpu_set_schedule(ems_gpu *h, int fused, int tile_rows, int x_chunks);
 
 /* CPML slabs of the tiled fused step (no reference counterpart): with
