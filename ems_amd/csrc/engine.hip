@@ -3826,7 +3826,8 @@ bool cpml_folded(const ems_gpu *h, int side, QuadCpml *cp = nullptr) {
 }
 
 // The quad kernels' geometry and grid.
-QuadGeom quad_geom(const ems_gpu *h, int side, bool cpf, unsigned *blocks) {
+QuadGeom quad_geom(const ems_gpu *h, int side, bool cpf, unsigned *blocks,
+                   unsigned *threads = nullptr) {
   QuadGeom g;
   g.nx = h->n[0], g.ny = h->n[1], g.nz = h->n[2];
   const int nq = (g.nz + 3) / 4;
@@ -3854,27 +3855,32 @@ QuadGeom quad_geom(const ems_gpu *h, int side, bool cpf, unsigned *blocks) {
   g.run = cached ? (int)((n + 7) / 8) : QUAD_RUN;
   const unsigned w = 8u * (unsigned)g.run;
   if (blocks) *blocks = (n + w - 1) / w * w;
+  // Planes whose quads fit fewer waves than four get blocks of those alone: a
+  // long line of small planes is bound by the waves it launches (100 000 x 1
+  // x 1 cells with CPML 274 to 160 us a step, x 8 x 8 361 to 222).
+  const int most = g.ny * std::max(g.nm, g.ql + g.qh);  // quads of a plane's larger part
+  if (threads) *threads = (unsigned)std::min(256, (most + 63) / 64 * 64);
   return g;
 }
 
 #define QUAD_LAUNCH(K)                                                                          \
   do {                                                                                          \
     if (h->oe && cpf)                                                                           \
-      hipLaunchKernelGGL((K<true, true>), dim3(nb), dim3(256), 0, h->stream, f, lanes_arg(h), g, cp); \
+      hipLaunchKernelGGL((K<true, true>), dim3(nb), dim3(nt), 0, h->stream, f, lanes_arg(h), g, cp); \
     else if (h->oe)                                                                             \
-      hipLaunchKernelGGL((K<true, false>), dim3(nb), dim3(256), 0, h->stream, f, lanes_arg(h), g, cp); \
+      hipLaunchKernelGGL((K<true, false>), dim3(nb), dim3(nt), 0, h->stream, f, lanes_arg(h), g, cp); \
     else if (cpf)                                                                               \
-      hipLaunchKernelGGL((K<false, true>), dim3(nb), dim3(256), 0, h->stream, f, lanes_arg(h), g, cp); \
+      hipLaunchKernelGGL((K<false, true>), dim3(nb), dim3(nt), 0, h->stream, f, lanes_arg(h), g, cp); \
     else                                                                                        \
-      hipLaunchKernelGGL((K<false, false>), dim3(nb), dim3(256), 0, h->stream, f, lanes_arg(h), g, cp); \
+      hipLaunchKernelGGL((K<false, false>), dim3(nb), dim3(nt), 0, h->stream, f, lanes_arg(h), g, cp); \
   } while (0)
 
 int launch_h(ems_gpu *h, const Fields &f) {
   if ((h->unfused_pf & 1) && quad_ok(h)) {
-    unsigned nb;
+    unsigned nb, nt;
     QuadCpml cp{};
     const bool cpf = cpml_folded(h, 0, &cp);
-    const QuadGeom g = quad_geom(h, 0, cpf, &nb);
+    const QuadGeom g = quad_geom(h, 0, cpf, &nb, &nt);
     QUAD_LAUNCH(h_update_quad);
     CK(h, hipGetLastError());
     return 0;
@@ -3893,10 +3899,10 @@ int launch_h(ems_gpu *h, const Fields &f) {
 
 int launch_e(ems_gpu *h, const Fields &f) {
   if ((h->unfused_pf & 2) && quad_ok(h)) {
-    unsigned nb;
+    unsigned nb, nt;
     QuadCpml cp{};
     const bool cpf = cpml_folded(h, 1, &cp);
-    const QuadGeom g = quad_geom(h, 1, cpf, &nb);
+    const QuadGeom g = quad_geom(h, 1, cpf, &nb, &nt);
     QUAD_LAUNCH(e_update_quad);
     CK(h, hipGetLastError());
     return 0;
