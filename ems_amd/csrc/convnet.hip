@@ -258,7 +258,8 @@ __device__ __forceinline__ T cn_uniform(const T *p, size_t i) {
 }
 
 // A causal convolution's sums over `ns` source channels and nine taps for
-// 64 samples and MW = 8 output channels per wave: out[m] = init[m] + sum_s
+// 64 samples and M output channels per wave (MW = 8, or 1 where that leaves
+// SIMDs idle: launch_fma): out[m] = init[m] + sum_s
 // sum_k w[s][k][m] src[s][t + off_k], channels and taps in order, one fused
 // multiply-add each (samples outside the sequence count as zeros; the
 // forward pass has off_k = -dil (8 - k), the input gradient +dil (8 - k)).
@@ -271,9 +272,10 @@ __device__ __forceinline__ T cn_uniform(const T *p, size_t i) {
 // a thread per output, which read its weights as bf16 from memory: 173).
 constexpr int MW = 8;
 constexpr int AHEAD = 4;  // source channels loaded ahead
+template <int M>
 __device__ __forceinline__ void cn_sums(const float *__restrict__ src, int ns,
                                         const float *__restrict__ w, int groups, int T, int dil,
-                                        int dir, unsigned t0, unsigned t, float acc[MW]) {
+                                        int dir, unsigned t0, unsigned t, float acc[M]) {
   // per tap: the lane's sample (clamped) and whether it is one; byte offsets
   // from the first sample that the wave may read, so that 32 bits hold them
   // for sequences of any length (and dilations below 2^27)
@@ -300,15 +302,15 @@ __device__ __forceinline__ void cn_sums(const float *__restrict__ src, int ns,
     for (int a = 0; a < AHEAD; a++) {
       const int c = c0 + a;
       if (c < ns) {
-        float wk[CN_K * MW];
+        float wk[CN_K * M];
         const float *wc = w + (size_t)c * groups * (CN_K * MW);
 #pragma unroll
-        for (int q = 0; q < CN_K * MW; q++) wk[q] = cn_uniform(wc, q);
+        for (int q = 0; q < CN_K * M; q++) wk[q] = cn_uniform(wc, q / M * MW + q % M);
 #pragma unroll
         for (int k = 0; k < CN_K; k++) {
           const float xv = in[k] ? x[a][k] : 0.0f;
 #pragma unroll
-          for (int m = 0; m < MW; m++) acc[m] += wk[k * MW + m] * xv;
+          for (int m = 0; m < M; m++) acc[m] += wk[k * M + m] * xv;
         }
         const float *nx = src + (size_t)(c + AHEAD < ns ? c + AHEAD : c) * T;
 #pragma unroll
@@ -319,13 +321,14 @@ __device__ __forceinline__ void cn_sums(const float *__restrict__ src, int ns,
 }
 
 // Grid of cn_fwd and cn_bwd: waves of 64 samples (4 a block), then sequences
-// and groups of 8 channels.
+// and groups of M channels.
 struct FmaArgs {
   const float *src;  // [b][ns][T]
   int ns;
   const float *w;  // [ns][groups of 8 output channels][9][8]
   int mc;          // output channels
-  int T, dil, tiles, groups;
+  int T, dil, tiles;
+  int groups, rows;    // groups of the grid's waves; of the weights (8 channels each)
   const float *bias;   // forward
   const float *h_in;   // forward: the residual input; gradient: gh of the layer above (or null)
   float *a, *out;      // forward: tanh, h (last layer: z); gradient: gh
@@ -333,29 +336,31 @@ struct FmaArgs {
   float *dz;             // gradient: dz of the layer below
   int last;              // forward: the last layer
 };
+template <int M>
 __device__ __forceinline__ void cn_place(const FmaArgs &p, int &b, int &m0, unsigned &t0) {
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const unsigned id = blockIdx.x * 4u + wv;
   const unsigned g = id % (unsigned)p.groups, q = id / (unsigned)p.groups;
   b = (int)(q / (unsigned)p.tiles);
   t0 = (q - (unsigned)b * (unsigned)p.tiles) * 64;
-  m0 = (int)g * MW;
+  m0 = (int)g * M;
 }
 
+template <int M>
 __global__ void __launch_bounds__(256) cn_fwd(FmaArgs p, int B) {
   int b, m0;
   unsigned t0;
-  cn_place(p, b, m0, t0);
+  cn_place<M>(p, b, m0, t0);
   if (b >= B) return;
   const unsigned t = t0 + (threadIdx.x & 63);
-  float acc[MW];
+  float acc[M];
 #pragma unroll
-  for (int m = 0; m < MW; m++) acc[m] = m0 + m < p.mc ? cn_uniform(p.bias, m0 + m) : 0.0f;
-  cn_sums(p.src + (size_t)b * p.ns * p.T, p.ns, p.w + m0 * CN_K, p.groups, p.T, p.dil, -1, t0, t,
-          acc);
+  for (int m = 0; m < M; m++) acc[m] = m0 + m < p.mc ? cn_uniform(p.bias, m0 + m) : 0.0f;
+  cn_sums<M>(p.src + (size_t)b * p.ns * p.T, p.ns, p.w + m0 / MW * (MW * CN_K) + m0 % MW, p.rows,
+             p.T, p.dil, -1, t0, t, acc);
   if (t >= (unsigned)p.T) return;
 #pragma unroll
-  for (int m = 0; m < MW; m++) {
+  for (int m = 0; m < M; m++) {
     if (m0 + m >= p.mc) continue;
     const size_t o = ((size_t)b * p.mc + m0 + m) * p.T + t;
     if (p.last) {
@@ -373,20 +378,21 @@ __global__ void __launch_bounds__(256) cn_fwd(FmaArgs p, int B) {
 
 // The gradient of a layer's input: gh = [gh +] sums, and dz = gh (1 - a^2)
 // of the layer below.
+template <int M>
 __global__ void __launch_bounds__(256) cn_bwd(FmaArgs p, int B) {
   int b, m0;
   unsigned t0;
-  cn_place(p, b, m0, t0);
+  cn_place<M>(p, b, m0, t0);
   if (b >= B) return;
   const unsigned t = t0 + (threadIdx.x & 63);
-  float acc[MW];
+  float acc[M];
 #pragma unroll
-  for (int m = 0; m < MW; m++) acc[m] = 0.0f;
-  cn_sums(p.src + (size_t)b * p.ns * p.T, p.ns, p.w + m0 * CN_K, p.groups, p.T, p.dil, 1, t0, t,
-          acc);
+  for (int m = 0; m < M; m++) acc[m] = 0.0f;
+  cn_sums<M>(p.src + (size_t)b * p.ns * p.T, p.ns, p.w + m0 / MW * (MW * CN_K) + m0 % MW, p.rows,
+             p.T, p.dil, 1, t0, t, acc);
   if (t >= (unsigned)p.T) return;
 #pragma unroll
-  for (int m = 0; m < MW; m++) {
+  for (int m = 0; m < M; m++) {
     if (m0 + m >= p.mc) continue;
     const size_t o = ((size_t)b * p.mc + m0 + m) * p.T + t;
     const float g = p.h_in ? p.h_in[o] + acc[m] : acc[m], v = p.a_below[o];
@@ -939,13 +945,24 @@ int predict(ems_cn *n, int B, int T) {
   return 0;
 }
 
+template <bool FWD, int M>
+void launch_fma_m(ems_cn *n, FmaArgs a, int B) {
+  a.groups = (a.mc + M - 1) / M;
+  const dim3 g((unsigned)(((size_t)B * a.tiles * a.groups + 3) / 4)), t(256);
+  if (FWD) hipLaunchKernelGGL(cn_fwd<M>, g, t, 0, n->stream, a, B);
+  else hipLaunchKernelGGL(cn_bwd<M>, g, t, 0, n->stream, a, B);
+}
+
 template <bool FWD>
 int launch_fma(ems_cn *n, FmaArgs a, int B) {
   a.tiles = (a.T - 1) / 64 + 1;
-  a.groups = (a.mc + MW - 1) / MW;
-  const dim3 g((unsigned)(((size_t)B * a.tiles * a.groups + 3) / 4)), t(256);
-  if (FWD) hipLaunchKernelGGL(cn_fwd, g, t, 0, n->stream, a, B);
-  else hipLaunchKernelGGL(cn_bwd, g, t, 0, n->stream, a, B);
+  a.rows = (a.mc + MW - 1) / MW;
+  // Fewer such waves than SIMDs: a wave per output channel, whose chain over
+  // the source channels is shorter (64 channels, 8 sequences of 512 samples
+  // 253 us a step against 335, 256 channels and one trace of 16 samples 769
+  // against 1138; at 1024 waves 379 against 374, at 2048 601 against 447).
+  if ((size_t)B * a.tiles * a.rows < 1024) launch_fma_m<FWD, 1>(n, a, B);
+  else launch_fma_m<FWD, MW>(n, a, B);
   CCK(n, hipGetLastError());
   return 0;
 }

@@ -161,11 +161,12 @@ def test_invalid_arguments():
 
 # Shapes at the edges of the convolutions' tiles: single samples and
 # channels, channels past and short of 16, 32 and 64, dilations that do not
-# divide the length, that exceed a block and that exceed the sequence, and
-# lengths around a block's 64 samples.
+# divide the length, that exceed a block and that exceed the sequence,
+# lengths around a block's 64 samples, and a batch that fills the chip (waves
+# of eight output channels in training; the others one).
 EDGES = [(1, 1, 1, (1, 1), 1, 1), (5, 3, 33, (3, 40), 2, 257), (4, 2, 48, (1, 2, 64, 100), 3, 130),
          (17, 18, 70, (7, 65, 200), 2, 96), (4, 2, 130, (2, 31), 1, 65), (2, 1, 32, (5, 1), 9, 63),
-         (4, 2, 64, (1, 2, 4, 8, 16, 32), 5, 500)]
+         (4, 2, 64, (1, 2, 4, 8, 16, 32), 5, 500), (5, 3, 52, (3, 40), 44, 257)]
 
 
 @pytest.mark.parametrize("shape", EDGES)
